@@ -107,8 +107,8 @@ typedef struct lxm_dn_pbuf {
 
 /* T forced tokens (device int32) through every layer without the head, in batches of LXM_DN_PB:
    the states and windows afterwards are those T calls of lxm_dn_step with these forced tokens
-   leave, bit for bit (each weight row is read once per batch; every sum keeps the step's
-   order). The stock generate's prefill role (the prompt before the first prediction, here with
+   leave, bit for bit (each weight row is read once per 64 tokens of a batch; every sum keeps the
+   step's order; lxm_dn_prefill_n takes larger batches). The stock generate's prefill role (the prompt before the first prediction, here with
    the decode's per-token arithmetic); a caller then steps from the next token. A token out of
    range sets *err = 1 (row 0 is used). Supports (hidden, live value dims, inter) = (2560, 4096,
    9216) or (256, 512, 512). Returns a hipError_t. */
@@ -119,7 +119,7 @@ int lxm_dn_prefill(const lxm_dn_params* p_host, const int32_t* tokens, int T,
    torch_chunk_gated_delta_rule, chunks of 64 from the prompt's first token) for T forced tokens
    through every layer without the head: each chunk of LXM_CHUNK (64) tokens goes through every
    layer, its delta rule as one call of lxm_gdn_chunk (include/lxm_chunk.h; MFMA), the row
-   kernels on its LXM_DN_PB-token slices. The projections, norms, conv, MLP and out_proj are
+   kernels on all of its tokens. The projections, norms, conv, MLP and out_proj are
    those of lxm_dn_prefill bit for bit on the same inputs; the delta rule's outputs and states
    are the chunked form's (equal to the recurrent step's up to the order of fp32 sums).
    buf's arrays hold LXM_CHUNK tokens (the sizes above with PB = 64) and buf->gl is set. The
@@ -127,6 +127,14 @@ int lxm_dn_prefill(const lxm_dn_params* p_host, const int32_t* tokens, int T,
    Returns a hipError_t. */
 int lxm_dn_prefill_chunked(const lxm_dn_params* p_host, const int32_t* tokens, int T,
                            const lxm_dn_pbuf* buf, void* stream);
+
+/* Both prompts with buffers of nt tokens (buf's arrays hold nt tokens each: the sizes above with
+   PB = nt): lxm_dn_prefill's results (chunked 0) or lxm_dn_prefill_chunked's (chunked 1; nt a
+   multiple of LXM_CHUNK, buf->gl set), in batches of nt tokens. A batch's rows run on the matrix
+   cores at any nt with the same bits; a larger nt reads each weight row fewer times. Returns a
+   hipError_t. */
+int lxm_dn_prefill_n(const lxm_dn_params* p_host, const int32_t* tokens, int T,
+                     const lxm_dn_pbuf* buf, int nt, int chunked, void* stream);
 
 #ifdef __cplusplus
 }

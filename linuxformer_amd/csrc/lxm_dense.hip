@@ -1344,18 +1344,15 @@ __global__ __launch_bounds__(NT, 1) void dn_run(const lxm_dn_params* __restrict_
 }
 
 // ---------------------------------------------------------------------------------------------
-// The batched prefill (lxm_dn_prefill): T forced tokens through every layer in batches of up to
-// PB tokens, without the head, leaving the states and windows that T calls of lxm_dn_step leave,
-// bit for bit. Per batch and layer: every token's input norm (pb_norm); the projections
-// (pb_rows: each weight row read once per batch; lane l sums its 64th of the row for every token
-// in the step's order, and the 64 lane sums of every (row, token) go through the step's pairwise
-// tree, spread over the lanes); every token's conv, l2norms, beta and decay (pb_prep: token t's
+// The batched prefill (lxm_dn_prefill, lxm_dn_prefill_n): T forced tokens through every layer in
+// batches, without the head, leaving the states and windows that T calls of lxm_dn_step leave, bit
+// for bit. Per batch and layer: every token's input norm (pb_norm); the projections (pb_mm: the
+// step's sums on the matrix cores); every token's conv, l2norms, beta and decay (pb_prep: token t's
 // window is the previous tokens' projections); the delta rule token by token (pb_gdn); the gated
-// norm and the windows' advance (pb_gnorm); out_proj (pb_hrows), the post norm, SwiGLU (pb_rows)
-// and down_proj (pb_hrows). The row kernels' inputs are stored in their weights' interleaved
-// order.
+// norm and the windows' advance (pb_gnorm); out_proj, the post norm, SwiGLU and down_proj (pb_mm).
+// The row kernels' inputs are stored in their weights' interleaved order.
 #define PB LXM_DN_PB
-#define PBT 256  // threads of the row kernels: 4 waves
+#define PBT 256
 
 // position of element c of a row of K = 64 G entries in the interleaved order
 __device__ __forceinline__ int il(int c, int G) {
@@ -1364,205 +1361,215 @@ __device__ __forceinline__ int il(int c, int G) {
   return ((k >> 3) * 64 + l) * 8 + (k & 7);
 }
 
-// V values per lane, each to be summed over the wave by the pairwise tree at offsets 32..1:
-// after the call lane l holds the sums of values l V / 64 .. + max(1, V / 64) - 1 (in v[0..]).
-// At offset o a lane keeps half of its values (the upper half where lane & o) and adds its
-// partner's partial sums of them: the same pairs as the tree's (lane l + lane l + o), since
-// fp32 addition is commutative.
-template <int V, int S>
-__device__ __forceinline__ void tree_scatter(float (&v)[V], int lane) {
-  if constexpr (S < 6) {
-    constexpr int o = 32 >> S, C = V >> S;
-    if constexpr (C >= 2) {
-      const bool up = (lane & o) != 0;
-#pragma unroll
-      for (int i = 0; i < C / 2; i++) {
-        const float send = up ? v[i] : v[i + C / 2];
-        const float keep = up ? v[i + C / 2] : v[i];
-        v[i] = keep + __shfl_xor(send, o);
-      }
-    } else {
-      v[0] = v[0] + __shfl_xor(v[0], o);
-    }
-    tree_scatter<V, S + 1>(v, lane);
-  }
-}
-
-// A chunk (CH = 8 or 4 bf16 values) of an interleaved bf16 row as 16 bytes
-template <int CH>
-__device__ __forceinline__ v4u chunk_bf(const uint16_t* row, int q, int lane) {
-  if constexpr (CH == 8) {
-    return reinterpret_cast<const v4u*>(row)[q * 64 + lane];
-  } else {
-    const uint2 u = reinterpret_cast<const uint2*>(row)[lane];
-    return v4u{u.x, u.y, 0u, 0u};
-  }
-}
-// acc += the chunk's products in entry order (bf16 x bf16 products are exact in fp32)
-template <int CH>
-__device__ __forceinline__ float chunk_dot(v4u w, v4u x, float acc) {
-#pragma unroll
-  for (int k = 0; k < CH / 2; k++) {
-    acc = __builtin_fmaf(bitsf(w[k] << 16), bitsf(x[k] << 16), acc);
-    acc = __builtin_fmaf(bitsf(w[k] & 0xffff0000u), bitsf(x[k] & 0xffff0000u), acc);
-  }
-  return acc;
-}
 __device__ __forceinline__ uint16_t bf16_bits(float v) { return (uint16_t)(fbits(v) >> 16); }
 
-// Rows for a batch of n <= PB tokens: the wave's R rows (MODE 2: R / 2 SwiGLU units, gate rows
-// from W and up rows from W2) over X (n x 64 G bf16, interleaved). The batch's inputs are staged
-// in LDS one chunk per lane at a time, double-buffered: each thread loads its share of chunk q + 1
-// into registers before chunk q's sums and stores it to LDS after them, so a chunk costs one
-// barrier and its loads overlap the arithmetic. MODE 0: out[b ldo + r] = D(s) (float); 1:
-// out[b ldo + r] = D(out + D(s)) (float, the residual); 2: out[b ldo + il(u, og)] =
-// D(D(silu(D(g))) * D(u)) (bf16).
-template <int G, int R, int MODE>
-__global__ __launch_bounds__(PBT) void pb_rows(const uint16_t* __restrict__ W,
-                                               const uint16_t* __restrict__ W2, int nrows,
-                                               const uint16_t* __restrict__ X, int n, void* out,
-                                               int ldo, int og) {
-  constexpr int CH = G == 4 ? 4 : 8, NC = G / CH, K = 64 * G, V = R * PB;
-  constexpr int RU = MODE == 2 ? R / 2 : R;  // distinct row indices per wave
-  constexpr int SPT = PB * 64 / PBT;         // staged chunks per thread
-  static_assert(MODE != 2 || (R % 2 == 0 && (V == 128 || V == 64)),
-                "units: gate and up sums 32 lanes apart");
-  __shared__ v4u xs[2][PB * 64];
-  const int lane = tid() & 63;
-  const int wv = blockIdx.x * (PBT / 64) + (tid() >> 6);
-  const uint16_t* rp[R];
+// Rows for a batch of n tokens on the fp32 matrix cores, in the step's order. The order of a dense
+// row is 64 groups of G entries, each summed in order from +0, then the pairwise tree over the
+// groups. v_mfma_f32_32x32x2_f32 accumulates its two k in order, each step one fused
+// multiply-add rounded to nearest even with denormals kept (checked against a host fmaf chain in
+// seven regimes of magnitude), and bf16 x bf16 products are exact in fp32: a group's chain of MFMAs
+// from zero is its sum, bit for bit, for 32 rows x 32 tokens at once.
+//
+// A workgroup (4 waves) takes 32 rows x 32 TN tokens. Its waves split the groups, not the tile: wave
+// w takes the groups congruent to w mod 4, so one step stages 4 consecutive groups' chunk q (64
+// bytes of each row and token) and every wave works on its own group of it. The 16 stages run in the
+// tree's order (m bit-reversed), so a wave's tree over its 16 groups is a binary counter of at
+// most 4 pending tiles; the last two levels join the 4 classes through LDS: (c0 + c2) + (c1 + c3).
+//
+// The bound is the fp32 matrix rate. A step is 4 (TN = 1) or 8 MFMAs of 64 cycles a wave; the loads
+// run PD + 2 steps ahead (PD of them in registers), the LDS buffers 2 steps, a wave's operands 1
+// step; two workgroups share a CU and cover each other's tree and barriers. Per layer of the
+// 2,560 / 4,096 / 9,216 stack at 2,048 tokens: SwiGLU 1.88 ms (103 TFLOP/s), projections 1.24, down_proj
+// 0.88 (110), out_proj 0.40; at 500 tokens 0.47, 0.32, 0.27 and 0.13 ms, where a wave per 8 rows x
+// 16 tokens on the vector unit (a fused multiply-add per term) took 1.08, 0.82, 0.81 and 0.42 (31
+// batches of 16). A product alone reaches 143 TFLOP/s with the operands' unpacking, two waves
+// a SIMD; without the staging 125, without the tree as well 130 (timed apart), the clock at
+// 2.15-2.2 GHz. Slower or no faster: 64 rows on 8 waves (one workgroup a CU: 0.34 and 0.17 ms for the
+// hidden rows at 500 tokens, the wide rows the same), the stages' tree one by one instead of in pairs
+// (twice the moves: 1.92 ms for SwiGLU at 2,048).
+// MODE 0: out[b ldo + r] = D(s) (float); 1: out[b ldo + r] = D(out + D(s)) (float, the residual);
+// 2 (SwiGLU, a tile's first half of rows from W, the second the same units from W2):
+// out[b ldo + il(u, og)] = D(D(silu(D(g))) * D(u)) (bf16).
+typedef float v16f __attribute__((ext_vector_type(16)));
+template <int G, int MODE, int TN>
+__global__ __launch_bounds__(PBT, 2) void pb_mm(const uint16_t* __restrict__ W,
+                                                const uint16_t* __restrict__ W2, int nrows,
+                                                const uint16_t* __restrict__ X, int n, void* out,
+                                                int ldo, int og, int ntt) {
+  constexpr int CH = G == 4 ? 4 : 8, NC = G / CH, K = 64 * G;
+  constexpr int PD = NC % 5 == 0 ? 5 : NC % 4 == 0 ? 4 : NC % 3 == 0 ? 3 : 1;  // loads' lead
+  constexpr int RT = 32, TT = 32 * TN, RU = MODE == 2 ? RT / 2 : RT;
+  constexpr int LN = RT + TT, TH = PBT, UN = 4 * LN, UPT = (UN + TH - 1) / TH;
+  constexpr int CS = LN + 4;      // a class's stride in 16-byte units (4 classes on 4 bank quarters)
+  constexpr int RS = RT + 4;      // the reduction's token stride in floats
+  constexpr int STG = 2 * 4 * CS * 16, RED = 4 * 32 * RS * 4;
+  static_assert(NC % PD == 0, "a stage's loop is unrolled by the lead");
+  __shared__ __align__(16) uint8_t sm[STG > RED ? STG : RED];
+  v4u* ring = reinterpret_cast<v4u*>(sm);
+  // (workgroups are dealt to the 8 XCDs in turn: a row tile's token tiles follow each other on one
+  // XCD, so its weights are fetched into one L2 once)
+  const int j8 = blockIdx.x >> 3, tt = j8 % ntt, rt = (j8 / ntt) * 8 + (blockIdx.x & 7);
+  const int r0 = rt * RU, b0 = tt * TT;
+  if (r0 >= nrows) return;
+  const int t = tid(), lane = t & 63, cls = wave_id();
+  // the units this thread stages: (line, class), lines 0 .. RT - 1 the rows, then the tokens
+  const uint16_t* src[UPT];
 #pragma unroll
-  for (int i = 0; i < R; i++) {
-    int r = wv * RU + i % RU;
-    r = r < nrows ? r : nrows - 1;  // (rows past the end load the last row, unused)
-    rp[i] = (MODE == 2 && i >= RU ? W2 : W) + (int64_t)r * K;
+  for (int i = 0; i < UPT; i++) {
+    const int u = t + i * TH, ln = u >> 2;
+    const uint16_t* base = X;
+    if (ln < RT) {
+      int r = r0 + (MODE == 2 ? ln % RU : ln);
+      r = r < nrows ? r : nrows - 1;  // (rows and tokens past the end: the last one's, unused)
+      base = (MODE == 2 && ln >= RU ? W2 : W) + (int64_t)r * K;
+    } else {
+      int b = b0 + ln - RT;
+      b = b < n ? b : n - 1;
+      base = X + (int64_t)b * K;
+    }
+    src[i] = base + (u & 3) * CH;
   }
-  // thread t stages (token, lane) = idx / 64, idx % 64 for idx = t + j PBT; tokens past n: zero
-  auto fetch = [&](int q, v4u (&st)[SPT]) {
+  const bool two = UN % TH == 0 || t + (UPT - 1) * TH < UN;  // (whole waves)
+  v4u st[PD][UPT];
+  int lq = 0, lst = 0;  // the next step to load: chunk lq of stage lst
+  auto load = [&](v4u (&s)[UPT]) {
+    const int m = ((lst & 1) << 3) | ((lst & 2) << 1) | ((lst & 4) >> 1) | ((lst & 8) >> 3);
+    const int off = (lq * 64 + 4 * m) * CH;
 #pragma unroll
-    for (int j = 0; j < SPT; j++) {
-      const int idx = tid() + j * PBT, b = idx >> 6;
-      st[j] = b < n ? chunk_bf<CH>(X + (int64_t)b * K, q, idx & 63) : v4u{0u, 0u, 0u, 0u};
+    for (int i = 0; i < UPT; i++) {
+      if (i + 1 < UPT || two) {
+        if constexpr (CH == 8) {
+          s[i] = *reinterpret_cast<const v4u*>(src[i] + off);
+        } else {
+          const uint2 v = *reinterpret_cast<const uint2*>(src[i] + off);
+          s[i] = v4u{v.x, v.y, 0u, 0u};
+        }
+      }
+    }
+    if (++lq == NC) {  // (past the last step: the last stage again, unused)
+      lq = 0;
+      lst = lst < 15 ? lst + 1 : 15;
     }
   };
-  float acc[R][PB];
+  auto stage = [&](const v4u (&s)[UPT], int p) {
 #pragma unroll
-  for (int i = 0; i < R; i++)
-#pragma unroll
-    for (int b = 0; b < PB; b++) acc[i][b] = 0.0f;
-  v4u st[SPT];
-  fetch(0, st);
-  for (int q = 0; q < NC; q++) {
-    v4u w[R];
-#pragma unroll
-    for (int i = 0; i < R; i++) w[i] = chunk_bf<CH>(rp[i], q, lane);
-    v4u* buf = xs[q & 1];
-#pragma unroll
-    for (int j = 0; j < SPT; j++) buf[tid() + j * PBT] = st[j];
-    // (every thread's share of chunk q is in; the buffer written next was last read two
-    // chunks ago, before this barrier)
-    lds_barrier();
-    if (q + 1 < NC) fetch(q + 1, st);
-#pragma unroll
-    for (int b = 0; b < PB; b++) {
-      const v4u xx = buf[b * 64 + lane];
-#pragma unroll
-      for (int i = 0; i < R; i++) acc[i][b] = chunk_dot<CH>(w[i], xx, acc[i][b]);
+    for (int i = 0; i < UPT; i++) {
+      const int u = t + i * TH;
+      if (i + 1 < UPT || two) ring[p * 4 * CS + (u & 3) * CS + (u >> 2)] = s[i];
     }
-  }
-  float v[V];
+  };
+  auto operands = [&](v4u (&f)[1 + TN], int p) {
+    const v4u* b = ring + p * 4 * CS + cls * CS;
+    f[0] = b[lane & 31];
 #pragma unroll
-  for (int i = 0; i < R; i++)
+    for (int i = 0; i < TN; i++) f[1 + i] = b[RT + 32 * i + (lane & 31)];
+  };
+  // lanes 0-31 hold the even k of a chunk's word, lanes 32-63 the odd: the bf16 half as a float
+  const uint32_t sel = lane < 32 ? 0x05040c0cu : 0x07060c0cu;
+  v16f acc[TN], p0[TN], p1[TN], p2[TN], p3[TN];
 #pragma unroll
-    for (int b = 0; b < PB; b++) v[i * PB + b] = acc[i][b];
-  tree_scatter<V, 0>(v, lane);
-  // (V < 64: 64 / V lanes hold each sum; the first of them stores it)
-  constexpr int PER = V >= 64 ? V / 64 : 1;
-  if (V < 64 && lane % (V < 64 ? 64 / V : 1) != 0) return;
+  for (int i = 0; i < TN; i++) p1[i] = p2[i] = p3[i] = v16f{0};
+  // steps 0 and 1 staged; steps 2 .. PD + 1 in flight, step s in slot s % PD
+  v4u f[1 + TN], s1[UPT];
+  load(st[0]);
+  load(s1);
+  stage(st[0], 0);
+  stage(s1, 1);
 #pragma unroll
-  for (int j = 0; j < PER; j++) {
-    const int vi = (lane * V) / 64 + j;
-    const int i = vi / PB, b = vi % PB;
-    if constexpr (MODE == 2) {
-      const float u = __shfl_xor(v[j], 32);  // (the up row's sum, 32 lanes on)
-      const int unit = wv * RU + i;
-      if (lane < 32 && unit < nrows && b < n)
-        static_cast<uint16_t*>(out)[(int64_t)b * ldo + il(unit, og)] =
-            bf16_bits(bf16r(silu_bf16(bf16r(v[j])) * bf16r(u)));
-    } else {
-      const int r = wv * RU + i;
-      if (r < nrows && b < n) {
-        float* o = static_cast<float*>(out) + (int64_t)b * ldo + r;
-        if constexpr (MODE == 0) *o = bf16r(v[j]);
-        else *o = bf16r(*o + bf16r(v[j]));
+  for (int d = 0; d < PD; d++) load(st[(d + 2) % PD]);
+  lds_barrier();
+  operands(f, 0);
+  int par = 0;  // the step's parity: its buffer
+  auto sum = [&](v16f (&c)[TN]) {  // one stage's NC steps: this wave's group, from zero
+#pragma unroll
+    for (int i = 0; i < TN; i++) c[i] = v16f{0};
+#pragma unroll
+    for (int q = 0; q < NC; q += PD) {
+#pragma unroll
+      for (int d = 0; d < PD; d++) {
+        // the next step's operands (staged before the last barrier); the step after that one
+        // into this step's buffer (read before the last barrier); this step's products
+        v4u fn[1 + TN];
+        operands(fn, par ^ 1);
+        stage(st[(d + 2) % PD], par);
+        load(st[(d + 2) % PD]);
+        __builtin_amdgcn_sched_barrier(0);  // (the reads first: they land under the products)
+#pragma unroll
+        for (int k = 0; k < CH / 2; k++) {
+          const float a = bitsf(__builtin_amdgcn_perm(f[0][k], 0u, sel));
+#pragma unroll
+          for (int i = 0; i < TN; i++)
+            c[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(
+                a, bitsf(__builtin_amdgcn_perm(f[1 + i][k], 0u, sel)), c[i], 0, 0, 0);
+        }
+        lds_barrier();
+#pragma unroll
+        for (int i = 0; i < 1 + TN; i++) f[i] = fn[i];
+        par ^= 1;
+      }
+    }
+  };
+  // stages in pairs, then the tree's counter over the pairs
+#pragma unroll 1
+  for (int sp = 0; sp < 8; sp++) {
+    sum(p0);
+    sum(acc);
+#pragma unroll
+    for (int i = 0; i < TN; i++) {
+      acc[i] = p0[i] + acc[i];
+      if (sp & 1) {
+        acc[i] = p1[i] + acc[i];
+        if (sp & 2) {
+          acc[i] = p2[i] + acc[i];
+          if (sp & 4) acc[i] = p3[i] + acc[i];
+          else p3[i] = acc[i];
+        } else {
+          p2[i] = acc[i];
+        }
+      } else {
+        p1[i] = acc[i];
       }
     }
   }
-}
-
-// Long rows (out_proj, down_proj: few rows of many entries) for a batch of PB tokens: the
-// workgroup's 4 waves share R rows, wave w taking tokens w BW .. w BW + BW - 1 (BW = PB / 4), each
-// wave reading its tokens' inputs straight from X (bf16; no LDS, no barriers: the rows are too
-// few to share a staged input among many waves), the next chunk's loads issued before this
-// chunk's sums. Sums and MODEs as pb_rows (0 and 1).
-template <int G, int R, int MODE>
-__global__ __launch_bounds__(PBT) void pb_hrows(const uint16_t* __restrict__ W, int nrows,
-                                                const uint16_t* __restrict__ X, int n, float* out,
-                                                int ldo) {
-  constexpr int CH = G == 4 ? 4 : 8, NC = G / CH, K = 64 * G, BW = PB / (PBT / 64), V = R * BW;
-  static_assert(V <= 64 && 64 % V == 0, "one sum per lane group");
-  const int lane = tid() & 63, wvl = tid() >> 6;
-  const int r0 = blockIdx.x * R, b0 = wvl * BW;
-  const uint16_t* rp[R];
+  // the classes' tiles through LDS, 32 tokens at a time (lane: rows 8 (i / 4) + 4 (lane / 32) +
+  // i % 4, token lane % 32); thread: 4 rows of one token
+  float* red = reinterpret_cast<float*>(sm);
 #pragma unroll
-  for (int i = 0; i < R; i++) {
-    const int r = r0 + i < nrows ? r0 + i : nrows - 1;
-    rp[i] = W + (int64_t)r * K;
-  }
-  const uint16_t* xp[BW];
+  for (int i = 0; i < TN; i++) {
+    lds_barrier();  // (the ring's, or the tokens' before: every wave has read it)
 #pragma unroll
-  for (int b = 0; b < BW; b++) {
-    const int bb = b0 + b < n ? b0 + b : n - 1;  // (tokens past n read token n - 1, unused)
-    xp[b] = X + (int64_t)bb * K;
-  }
-  float acc[R][BW];
+    for (int r = 0; r < 4; r++)
+      *reinterpret_cast<v4f*>(red + (cls * 32 + (lane & 31)) * RS + 8 * r + 4 * (lane >> 5)) =
+          v4f{acc[i][4 * r], acc[i][4 * r + 1], acc[i][4 * r + 2], acc[i][4 * r + 3]};
+    lds_barrier();
+    auto sum4 = [&](int tok, int r) {
+      const v4f* c = reinterpret_cast<const v4f*>(red + tok * RS + r);
+      constexpr int S = 32 * RS / 4;
+      return (c[0] + c[2 * S]) + (c[S] + c[3 * S]);
+    };
+    if constexpr (MODE == 2) {
+      const int tok = t / (RU / 4), r = 4 * (t % (RU / 4)), b = b0 + 32 * i + tok, u = r0 + r;
+      if (tok < 32 && b < n && u < nrows) {
+        const v4f g = sum4(tok, r), up = sum4(tok, RU + r);
+        uint16_t* o = static_cast<uint16_t*>(out) + (int64_t)b * ldo;
 #pragma unroll
-  for (int i = 0; i < R; i++)
+        for (int k = 0; k < 4; k++)
+          if (u + k < nrows)
+            o[il(u + k, og)] = bf16_bits(bf16r(silu_bf16(bf16r(g[k])) * bf16r(up[k])));
+      }
+    } else {
+      const int tok = t / (RT / 4), r = 4 * (t % (RT / 4)), b = b0 + 32 * i + tok;
+      if (b < n) {
+        const v4f v = sum4(tok, r);
+        float* o = static_cast<float*>(out) + (int64_t)b * ldo + r0 + r;
 #pragma unroll
-    for (int b = 0; b < BW; b++) acc[i][b] = 0.0f;
-  v4u w[R], x[BW];
-#pragma unroll
-  for (int i = 0; i < R; i++) w[i] = chunk_bf<CH>(rp[i], 0, lane);
-#pragma unroll
-  for (int b = 0; b < BW; b++) x[b] = chunk_bf<CH>(xp[b], 0, lane);
-  for (int q = 0; q < NC; q++) {
-    v4u wn[R], xn[BW];
-    const int qn = q + 1 < NC ? q + 1 : q;  // (the last chunk reloads itself, unused)
-#pragma unroll
-    for (int i = 0; i < R; i++) wn[i] = chunk_bf<CH>(rp[i], qn, lane);
-#pragma unroll
-    for (int b = 0; b < BW; b++) xn[b] = chunk_bf<CH>(xp[b], qn, lane);
-#pragma unroll
-    for (int b = 0; b < BW; b++)
-#pragma unroll
-      for (int i = 0; i < R; i++) acc[i][b] = chunk_dot<CH>(w[i], x[b], acc[i][b]);
-#pragma unroll
-    for (int i = 0; i < R; i++) w[i] = wn[i];
-#pragma unroll
-    for (int b = 0; b < BW; b++) x[b] = xn[b];
-  }
-  float v[V];
-#pragma unroll
-  for (int i = 0; i < R; i++)
-#pragma unroll
-    for (int b = 0; b < BW; b++) v[i * BW + b] = acc[i][b];
-  tree_scatter<V, 0>(v, lane);
-  if (lane % (64 / V) != 0) return;  // (64 / V lanes hold each sum; the first stores it)
-  const int vi = (lane * V) / 64, i = vi / BW, b = b0 + vi % BW, r = r0 + i;
-  if (r < nrows && b < n) {
-    float* o = out + (int64_t)b * ldo + r;
-    if constexpr (MODE == 0) *o = bf16r(v[0]);
-    else *o = bf16r(*o + bf16r(v[0]));
+        for (int k = 0; k < 4; k++)
+          if (r0 + r + k < nrows) {
+            if constexpr (MODE == 0) o[k] = bf16r(v[k]);
+            else o[k] = bf16r(o[k] + bf16r(v[k]));
+          }
+      }
+    }
   }
 }
 
@@ -1945,136 +1952,117 @@ extern "C" int lxm_dn_run(const lxm_dn_params* ph, const lxm_dn_params* pd, int 
   return (int)hipErrorInvalidValue;
 }
 
-// the batched prefill's row kernels: R rows per wave (MODE 2: R / 2 units), 4 waves per workgroup
-template <int G, int R, int MODE>
+// the batched prefill's row kernels (MODE 2: nrows units of W and W2): 64 tokens a workgroup share
+// its rows' unpacking (two products an operand); up to 32 tokens take one 32-token tile, with half
+// the registers and four workgroups a CU to stream the weights
+template <int G, int MODE, int TN>
+static void launch_mm(const uint16_t* W, const uint16_t* W2, int nrows, const uint16_t* X, int n,
+                      void* out, int ldo, int og, hipStream_t st) {
+  constexpr int RU = MODE == 2 ? 16 : 32;
+  const int nrt = (nrows + RU - 1) / RU, ntt = (n + 32 * TN - 1) / (32 * TN);
+  hipLaunchKernelGGL((pb_mm<G, MODE, TN>), dim3((nrt + 7) / 8 * 8 * ntt), dim3(PBT), 0, st, W, W2,
+                     nrows, X, n, out, ldo, og, ntt);
+}
+template <int G, int MODE>
 static void launch_pb(const uint16_t* W, const uint16_t* W2, int nrows, const uint16_t* X, int n,
                       void* out, int ldo, int og, hipStream_t st) {
-  const int per = (PBT / 64) * (MODE == 2 ? R / 2 : R);
-  hipLaunchKernelGGL((pb_rows<G, R, MODE>), dim3((nrows + per - 1) / per), dim3(PBT), 0, st, W, W2,
-                     nrows, X, n, out, ldo, og);
+  if (n <= 32) launch_mm<G, MODE, 1>(W, W2, nrows, X, n, out, ldo, og, st);
+  else launch_mm<G, MODE, 2>(W, W2, nrows, X, n, out, ldo, og, st);
 }
-// the residual's long rows: 8 rows per workgroup, the batch's tokens split over its 4 waves
-template <int G>
-static void launch_hrows(const uint16_t* W, int nrows, const uint16_t* X, int n, float* out, int ldo,
-                         hipStream_t st) {
-  constexpr int R = 8;
-  hipLaunchKernelGGL((pb_hrows<G, R, 1>), dim3((nrows + R - 1) / R), dim3(PBT), 0, st, W, nrows, X,
-                     n, out, ldo);
-}
-// (G of the hidden rows, live value dims, inter) = (40, 64, 144) or (4, 8, 8)
+// (G of the hidden rows, live value dims, inter) = (40, 64, 144) or (4, 8, 8). A batch's delta rule
+// runs token by token (pb_gdn on PB-token slices), or chunk by chunk (chunked: lxm_gdn_chunk, the
+// batch a whole number of chunks from the prompt's first token but for the prompt's end).
 template <int GH, int GV, int GI>
-static void pb_layer(const lxm_dn_params* ph, const lxm_dn_layer& ly, const lxm_dn_pbuf* pb, int n,
-                     hipStream_t st) {
+static hipError_t pb_layer(const lxm_dn_params* ph, const lxm_dn_layer& ly, const lxm_dn_pbuf* pb,
+                           int n, bool chunked, hipStream_t st) {
   const int H = ph->hidden, I = ph->inter, nk = ph->nk, kl = ph->kl, rl = ph->rl, R = ph->nv / nk;
   const int nq = nk * kl, nvr = nk * rl * VD, nproj = 2 * nq + 2 * nvr + 2 * nk * rl;
   const float eps = ph->rms_eps;
   hipLaunchKernelGGL(pb_norm, dim3(n), dim3(NT), 0, st, pb->h, ly.ln_in, eps, H, GH, pb->xn);
-  launch_pb<GH, 8, 0>(ly.proj, nullptr, nproj, pb->xn, n, pb->P, nproj, 0, st);
+  launch_pb<GH, 0>(ly.proj, nullptr, nproj, pb->xn, n, pb->P, nproj, 0, st);
   const PbGdn g{ly.conv_qk, ly.conv_v, ly.A_log, ly.dt_bias, ly.rec, ly.conv, pb->P, pb->qk,
-                pb->v, pb->g, pb->live, pb->o, nk, kl, rl, R, nproj, n, nullptr};
+                pb->v, pb->g, pb->live, pb->o, nk, kl, rl, R, nproj, n,
+                chunked ? pb->gl : nullptr};
   hipLaunchKernelGGL(pb_prep, dim3(n, nk), dim3(KD), 0, st, g);
-  hipLaunchKernelGGL(pb_gdn, dim3(nk * rl * QC), dim3(NT), 0, st, g);
-  hipLaunchKernelGGL(pb_gnorm, dim3(n), dim3(PBT), 0, st, pb->o, pb->P, nproj, 2 * nq + nvr,
-                     ly.gnorm, ph->geps, nk * rl, GV, pb->ys, ly.conv, n, nk, kl, rl, R);
-  launch_hrows<GV>(ly.out, H, pb->ys, n, pb->h, H, st);
-  hipLaunchKernelGGL(pb_norm, dim3(n), dim3(NT), 0, st, pb->h, ly.ln_post, eps, H, GH, pb->xn);
-  // (SwiGLU: 2 units per wave, 1,152 workgroups at 3 per CU; with 4 units per wave its 576
-  // workgroups took two rounds of 512, 44 us against 34)
-  launch_pb<GH, 4, 2>(ly.gate, ly.up, I, pb->xn, n, pb->act, I, GI, st);
-  launch_hrows<GI>(ly.down, H, pb->act, n, pb->h, H, st);
-}
-
-extern "C" int lxm_dn_prefill(const lxm_dn_params* ph, const int32_t* tokens, int T,
-                              const lxm_dn_pbuf* pb, void* stream) {
-  if (!dims_ok(ph) || !pb || !tokens || T < 0) return (int)hipErrorInvalidValue;
-  const int gh = g_of(ph->hidden), gv = g_of(ph->nk * ph->rl * VD), gi = g_of(ph->inter);
-  const bool full = gh == 40 && gv == 64 && gi == 144, small = gh == 4 && gv == 8 && gi == 8;
-  if (!full && !small) return (int)hipErrorInvalidValue;
-  hipStream_t st = (hipStream_t)stream;
-  for (int b0 = 0; b0 < T; b0 += PB) {
-    const int n = T - b0 < PB ? T - b0 : PB;
-    hipLaunchKernelGGL(pb_embed, dim3(n), dim3(PBT), 0, st, ph->embed, tokens + b0, ph->hidden,
-                       ph->vocab, pb->h, ph->err);
-    for (int L = 0; L < ph->n_layers; L++) {
-      if (full) pb_layer<40, 64, 144>(ph, ph->layers_host[L], pb, n, st);
-      else pb_layer<4, 8, 8>(ph, ph->layers_host[L], pb, n, st);
+  if (chunked) {
+    lxm_chunk_io io;
+    io.qk_ts = (int64_t)nk * 2 * KD;
+    io.qk_hs = 2 * KD;
+    io.v_ts = nvr;
+    io.g_ts = 2 * (int64_t)nk * rl;
+    io.g_hs = 2;
+    io.gl_ts = (int64_t)nk * rl;
+    io.o_ts = nvr;
+    io.S = ly.rec;
+    io.n_slots = nk * rl;
+    io.rl = rl;
+    io.rfull = R;
+    io.kl = kl;
+    io.o_bf16 = 1;
+    for (int s = 0; s < n; s += LXM_CHUNK) {
+      io.q = pb->qk + s * io.qk_ts;
+      io.k = io.q + KD;
+      io.v = pb->v + s * io.v_ts;
+      io.beta = pb->g + s * io.g_ts;
+      io.g = pb->gl + s * io.gl_ts;
+      io.o = pb->o + s * io.o_ts;
+      io.n = n - s < LXM_CHUNK ? n - s : LXM_CHUNK;
+      const int e = lxm_gdn_chunk(&io, st);
+      if (e) return (hipError_t)e;
+    }
+  } else {
+    for (int s = 0; s < n; s += PB) {
+      PbGdn gs = g;
+      gs.n = n - s < PB ? n - s : PB;
+      gs.qk += (int64_t)s * nk * 2 * KD;
+      gs.v += (int64_t)s * nvr;
+      gs.g += (int64_t)s * nk * rl * 2;
+      gs.live += (int64_t)s * nk * 2;
+      gs.o += (int64_t)s * nvr;
+      hipLaunchKernelGGL(pb_gdn, dim3(nk * rl * QC), dim3(NT), 0, st, gs);
     }
   }
-  return (int)hipGetLastError();
-}
-
-// The stock forward's prompt (the T > 1 path: Qwen3_5GatedDeltaNet.forward :517-529 calls
-// torch_chunk_gated_delta_rule): super-batches of up to LXM_CHUNK tokens, each a chunk of the
-// chunked delta rule (lxm_gdn_chunk, MFMA), the row kernels run on its PB-token slices. Every
-// other sum keeps the step's order; the delta rule's outputs and states are the chunked form's.
-template <int GH, int GV, int GI>
-static hipError_t pc_layer(const lxm_dn_params* ph, const lxm_dn_layer& ly, const lxm_dn_pbuf* pb,
-                           int n, hipStream_t st) {
-  const int H = ph->hidden, I = ph->inter, nk = ph->nk, kl = ph->kl, rl = ph->rl, R = ph->nv / nk;
-  const int nq = nk * kl, nvr = nk * rl * VD, nproj = 2 * nq + 2 * nvr + 2 * nk * rl;
-  const float eps = ph->rms_eps;
-  hipLaunchKernelGGL(pb_norm, dim3(n), dim3(NT), 0, st, pb->h, ly.ln_in, eps, H, GH, pb->xn);
-  for (int s = 0; s < n; s += PB)
-    launch_pb<GH, 8, 0>(ly.proj, nullptr, nproj, pb->xn + (int64_t)s * H, n - s < PB ? n - s : PB,
-                        pb->P + (int64_t)s * nproj, nproj, 0, st);
-  const PbGdn g{ly.conv_qk, ly.conv_v, ly.A_log, ly.dt_bias, ly.rec, ly.conv, pb->P, pb->qk,
-                pb->v, pb->g, pb->live, pb->o, nk, kl, rl, R, nproj, n, pb->gl};
-  hipLaunchKernelGGL(pb_prep, dim3(n, nk), dim3(KD), 0, st, g);
-  lxm_chunk_io io;
-  io.q = pb->qk;
-  io.k = pb->qk + KD;
-  io.v = pb->v;
-  io.beta = pb->g;
-  io.g = pb->gl;
-  io.S = ly.rec;
-  io.o = pb->o;
-  io.qk_ts = (int64_t)nk * 2 * KD;
-  io.qk_hs = 2 * KD;
-  io.v_ts = nvr;
-  io.g_ts = 2 * (int64_t)nk * rl;
-  io.g_hs = 2;
-  io.gl_ts = (int64_t)nk * rl;
-  io.o_ts = nvr;
-  io.n = n;
-  io.n_slots = nk * rl;
-  io.rl = rl;
-  io.rfull = R;
-  io.kl = kl;
-  io.o_bf16 = 1;
-  const int e = lxm_gdn_chunk(&io, st);
-  if (e) return (hipError_t)e;
   hipLaunchKernelGGL(pb_gnorm, dim3(n), dim3(PBT), 0, st, pb->o, pb->P, nproj, 2 * nq + nvr,
                      ly.gnorm, ph->geps, nk * rl, GV, pb->ys, ly.conv, n, nk, kl, rl, R);
-  for (int s = 0; s < n; s += PB)
-    launch_hrows<GV>(ly.out, H, pb->ys + (int64_t)s * nvr, n - s < PB ? n - s : PB,
-                     pb->h + (int64_t)s * H, H, st);
+  launch_pb<GV, 1>(ly.out, nullptr, H, pb->ys, n, pb->h, H, 0, st);
   hipLaunchKernelGGL(pb_norm, dim3(n), dim3(NT), 0, st, pb->h, ly.ln_post, eps, H, GH, pb->xn);
-  for (int s = 0; s < n; s += PB)
-    launch_pb<GH, 4, 2>(ly.gate, ly.up, I, pb->xn + (int64_t)s * H, n - s < PB ? n - s : PB,
-                        pb->act + (int64_t)s * I, I, GI, st);
-  for (int s = 0; s < n; s += PB)
-    launch_hrows<GI>(ly.down, H, pb->act + (int64_t)s * I, n - s < PB ? n - s : PB,
-                     pb->h + (int64_t)s * H, H, st);
+  launch_pb<GH, 2>(ly.gate, ly.up, I, pb->xn, n, pb->act, I, GI, st);
+  launch_pb<GI, 1>(ly.down, nullptr, H, pb->act, n, pb->h, H, 0, st);
   return hipGetLastError();
 }
 
-extern "C" int lxm_dn_prefill_chunked(const lxm_dn_params* ph, const int32_t* tokens, int T,
-                                      const lxm_dn_pbuf* pb, void* stream) {
-  if (!dims_ok(ph) || !pb || !pb->gl || !tokens || T < 0 || ph->kl > 128 || ph->kl % 16)
+extern "C" int lxm_dn_prefill_n(const lxm_dn_params* ph, const int32_t* tokens, int T,
+                                const lxm_dn_pbuf* pb, int nt, int chunked, void* stream) {
+  if (!dims_ok(ph) || !pb || !tokens || T < 0 || nt < 1) return (int)hipErrorInvalidValue;
+  if (chunked && (!pb->gl || ph->kl > 128 || ph->kl % 16 || nt % LXM_CHUNK))
     return (int)hipErrorInvalidValue;
   const int gh = g_of(ph->hidden), gv = g_of(ph->nk * ph->rl * VD), gi = g_of(ph->inter);
   const bool full = gh == 40 && gv == 64 && gi == 144, small = gh == 4 && gv == 8 && gi == 8;
   if (!full && !small) return (int)hipErrorInvalidValue;
   hipStream_t st = (hipStream_t)stream;
-  for (int b0 = 0; b0 < T; b0 += LXM_CHUNK) {
-    const int n = T - b0 < LXM_CHUNK ? T - b0 : LXM_CHUNK;
+  for (int b0 = 0; b0 < T; b0 += nt) {
+    const int n = T - b0 < nt ? T - b0 : nt;
     hipLaunchKernelGGL(pb_embed, dim3(n), dim3(PBT), 0, st, ph->embed, tokens + b0, ph->hidden,
                        ph->vocab, pb->h, ph->err);
     for (int L = 0; L < ph->n_layers; L++) {
-      const hipError_t e = full ? pc_layer<40, 64, 144>(ph, ph->layers_host[L], pb, n, st)
-                                : pc_layer<4, 8, 8>(ph, ph->layers_host[L], pb, n, st);
+      const lxm_dn_layer& ly = ph->layers_host[L];
+      const hipError_t e = full ? pb_layer<40, 64, 144>(ph, ly, pb, n, chunked != 0, st)
+                                : pb_layer<4, 8, 8>(ph, ly, pb, n, chunked != 0, st);
       if (e != hipSuccess) return (int)e;
     }
   }
   return (int)hipGetLastError();
+}
+
+extern "C" int lxm_dn_prefill(const lxm_dn_params* ph, const int32_t* tokens, int T,
+                              const lxm_dn_pbuf* pb, void* stream) {
+  return lxm_dn_prefill_n(ph, tokens, T, pb, PB, 0, stream);
+}
+
+// The stock forward's prompt (the T > 1 path: Qwen3_5GatedDeltaNet.forward :517-529 calls
+// torch_chunk_gated_delta_rule): every other sum keeps the step's order; the delta rule's outputs
+// and states are the chunked form's.
+extern "C" int lxm_dn_prefill_chunked(const lxm_dn_params* ph, const int32_t* tokens, int T,
+                                      const lxm_dn_pbuf* pb, void* stream) {
+  return lxm_dn_prefill_n(ph, tokens, T, pb, LXM_CHUNK, 1, stream);
 }

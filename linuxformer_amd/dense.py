@@ -36,8 +36,8 @@ class DnPbuf(ctypes.Structure):
     _fields_ = [(n, P64) for n in ("h", "xn", "P", "qk", "v", "g", "live", "o", "ys", "act", "gl")]
 
 
-PB = 16  # tokens per prefill batch (LXM_DN_PB)
 CHUNK = 64  # tokens per chunk of the chunked prompt (LXM_CHUNK)
+NT_MAX = 2048  # tokens per prompt batch at most (~155 KB of buffers a token at config 4)
 
 
 class DnParams(ctypes.Structure):
@@ -118,7 +118,7 @@ class DenseDecode:
         self.forced = torch.zeros(max_steps, dtype=torch.int32, device=dev)
         self.max_steps = max_steps
         self.graph = None
-        self._pb = None
+        self._pb, self._pb_nt = None, 0
 
     def _params(self, n_forced: int, prof: int = 0):
         sp, d = self.spec, self.dims
@@ -136,34 +136,32 @@ class DenseDecode:
         pd = torch.frombuffer(bytearray(bytes(p)), dtype=torch.uint8).to(self.dev)
         return p, pd
 
-    def _pbuf(self, chunked: bool = False):
-        """The prompt's buffers (allocated on first use): PB tokens for the batched prefill,
-        CHUNK tokens (and the log decays) for the chunked one."""
-        key = "_pbc" if chunked else "_pb"
-        if getattr(self, key, None) is None:
+    def _pbuf(self, T: int):
+        """The prompt's buffers and the tokens they hold: whole chunks, enough for T tokens up to
+        NT_MAX (allocated on first use, again for a longer prompt)."""
+        nt = min(NT_MAX, (T + CHUNK - 1) // CHUNK * CHUNK)
+        if self._pb is None or self._pb_nt < nt:
             sp = self.spec
             H, nk, rl, I = sp.hidden, sp.nk, sp.r_live, sp.inter
             nvr = nk * rl * 128
             sizes = dict(h=H, xn=H, P=self.nproj, qk=nk * 2 * 256, v=nvr, g=nk * rl * 2,
-                         live=nk * 2, o=nvr, ys=nvr, act=I)
-            if chunked:
-                sizes["gl"] = nk * rl
+                         live=nk * 2, o=nvr, ys=nvr, act=I, gl=nk * rl)
             bf = ("xn", "ys", "act")  # (the row kernels' inputs, bf16)
-            nt = CHUNK if chunked else PB
-            ts = {k: torch.zeros(nt * n, device=self.dev,
-                                 dtype=torch.bfloat16 if k in bf else torch.float32)
-                  for k, n in sizes.items()}
-            setattr(self, key + "_t", ts)
-            setattr(self, key, DnPbuf(**{k: t.data_ptr() for k, t in ts.items()}))
-        return getattr(self, key)
+            self._pb = None  # (the smaller set is given back first)
+            self._pb_t = {k: torch.empty(nt * n, device=self.dev,
+                                         dtype=torch.bfloat16 if k in bf else torch.float32)
+                          for k, n in sizes.items()}
+            self._pb = DnPbuf(**{k: t.data_ptr() for k, t in self._pb_t.items()})
+            self._pb_nt = nt
+        return self._pb, self._pb_nt
 
     def prefill(self, tokens, mode: str = "batched") -> None:
         """The tokens through every layer without the head; no predictions are made. A caller
         then steps from the next token: run([next], n).
 
-        mode "batched" (lxm_dn_prefill: batches of PB tokens, each weight row read once per
-        batch): the cache's states and windows afterwards are those of len(tokens) forced steps
-        of run(), bit for bit. mode "chunked" (lxm_dn_prefill_chunked): the stock forward's
+        mode "batched" (lxm_dn_prefill_n: batches of up to NT_MAX tokens, each layer's products on
+        the matrix cores in the step's order): the cache's states and windows afterwards are those of len(tokens) forced steps
+        of run(), bit for bit. mode "chunked": the stock forward's
         T > 1 path, the delta rule in chunks of 64 on the matrix cores
         (torch_chunk_gated_delta_rule); every other sum as in "batched", the delta rule's outputs
         and states those of the chunked form."""
@@ -175,13 +173,13 @@ class DenseDecode:
         if int(t.min()) < 0 or int(t.max()) >= self.spec.vocab:
             raise ValueError("prefill token out of range")
         chunked = mode == "chunked"
-        pb = self._pbuf(chunked)
+        pb, nt = self._pbuf(int(t.numel()))
         tok = t.to(torch.int32).to(self.dev)
         self.err.zero_()
         p, _ = self._params(1)
         st = ctypes.c_void_p(torch.cuda.current_stream(self.dev).cuda_stream)
-        fn = self.lib.lxm_dn_prefill_chunked if chunked else self.lib.lxm_dn_prefill
-        e = fn(ctypes.byref(p), ctypes.c_void_p(tok.data_ptr()), int(t.numel()), ctypes.byref(pb), st)
+        e = self.lib.lxm_dn_prefill_n(ctypes.byref(p), ctypes.c_void_p(tok.data_ptr()),
+                                      int(t.numel()), ctypes.byref(pb), nt, int(chunked), st)
         if e:
             raise RuntimeError(f"dense prefill launch failed: hipError {e}")
         torch.cuda.synchronize(self.dev)

@@ -145,6 +145,50 @@ def test_dense_prefill_small(cuda, T, seed):
     check_prefill(T, 6, seed=seed)
 
 
+@pytest.mark.parametrize("n", [1, 32, 33, 64, 65, 97])
+def test_dense_prefill_token_tiles(cuda, n):
+    """Prompts at the row kernels' token tiles (32 tokens in one tile, 64 a workgroup beyond): a
+    whole tile, one past it, one token alone, a last workgroup of one tile and a token."""
+    check_prefill(n + 1, 2, seed=3)
+
+
+@pytest.mark.parametrize("chunked,nt", [(0, 16), (0, 48), (1, 64), (1, 128)])
+def test_dense_prefill_batches(cuda, chunked, nt):
+    """The C entries with buffers of nt tokens (16 and 64: lxm_dn_prefill and
+    lxm_dn_prefill_chunked; other sizes: lxm_dn_prefill_n) leave the same bits as one batch of the
+    whole prompt: 150 tokens, so that every size has a partial last batch."""
+    import ctypes
+
+    spec, dm_cpu, _ = model()
+    conv0, rec0 = synth.dense_state(dm_cpu, 3)
+    toks = [int(x) for x in np.random.default_rng(31).integers(0, spec.vocab, 150)]
+    print(f"[gpu-test] dense prefill batches: chunked={chunked} nt={nt}", flush=True)
+    dm = synth.dense_to(dm_cpu, "cuda")
+    out = []
+    for whole in (True, False):
+        cache = fast.StateCache(conv0, rec0, "bf16", "cuda")
+        dd = dense.DenseDecode(dm, cache)
+        if whole:
+            dd.prefill(toks, mode="chunked" if chunked else "batched")
+        else:
+            pb, _ = dd._pbuf(nt)
+            tok = torch.tensor(toks, dtype=torch.int32, device="cuda")
+            p, _ = dd._params(1)
+            args = [ctypes.byref(p), ctypes.c_void_p(tok.data_ptr()), len(toks), ctypes.byref(pb)]
+            st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+            if nt == 16:
+                e = dd.lib.lxm_dn_prefill(*args, st)
+            elif nt == 64:
+                e = dd.lib.lxm_dn_prefill_chunked(*args, st)
+            else:
+                e = dd.lib.lxm_dn_prefill_n(*args, nt, chunked, st)
+            assert e == 0
+            torch.cuda.synchronize()
+        out.append((cache.conv_numpy(), cache.rec_numpy()))
+    for a, b in zip(*out):
+        assert (bits(a) == bits(b)).all()
+
+
 def test_dense_prefill_full_widths(cuda):
     check_prefill(21, 3, seed=5, name="mid")
 
