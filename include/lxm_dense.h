@@ -98,7 +98,8 @@ typedef struct lxm_dn_pbuf {
   float* qk;   /* (PB, nk, 2, 256): the normed query (times 1/16) and key */
   float* v;    /* (PB, nk x rl x 128): the values after the conv */
   float* g;    /* (PB, nk x rl, 2): beta and exp(g) */
-  float* live; /* (PB, nk, 2): 1 where the query / key has a nonzero element */
+  float* live; /* (PB, nk, 2): 0 where the query / key is all zero, 2 where every live dim's
+                  normed element is nonzero, else 1 */
   float* o;    /* (PB, nk x rl x 128): the delta rule's outputs */
   uint16_t* ys;  /* (PB, nk x rl x 128) bf16: the gated norm's output, interleaved */
   uint16_t* act; /* (PB, inter) bf16: SwiGLU's output, interleaved */

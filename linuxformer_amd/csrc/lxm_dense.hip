@@ -1678,88 +1678,133 @@ __global__ __launch_bounds__(KD) void pb_prep(PbGdn a) {
     const bool any = __ballot(nz) != 0ull;
     ss = bf16r(sum64(ss));
     const float inv = bf16r(rsqrt_(bf16r(ss + 1e-6f)));
+    bool zero = false;  // a live dim's normed element that is zero
 #pragma unroll
     for (int i = 0; i < 4; i++) {
       float v = bf16r(xs[i] * inv);
       if (!wv) v = v * 0.0625f;
       o[lane + 64 * i] = v;
+      zero |= lane + 64 * i < kl && v == 0.0f;
     }
-    if (lane == 0) a.live[((int64_t)b * nk + kh) * 2 + wv] = any ? 1.0f : 0.0f;
+    const bool all = __ballot(zero) == 0ull;
+    if (lane == 0)
+      a.live[((int64_t)b * nk + kh) * 2 + wv] = !any ? 0.0f : all ? 2.0f : 1.0f;
   }
 }
-// the delta rule of one live value head's 32 state columns (nk x rl x QC workgroups, as the
-// step's) over the batch's tokens in order, the tile in registers throughout
-struct PbLds {
-  float qk[PB][2][KD];
-  float vb[PB][QW], bg[PB][2], lv[PB];
-  float bsk[16 * QW], bso[16 * QW], dl[QW];
+// x summed over the NB lanes of a column in lane order, on every one of them: lane b adds its left
+// neighbour's running sum to its own x, NB - 1 times (after k steps lane b holds x[b - k] + .. + x[b] in
+// order, so the column's last lane ends with the whole sum), then that lane's value is spread.
+// DPP moves on the vector unit, no LDS round trip.
+template <int NB>
+__device__ __forceinline__ float col_last(float x) {
+  float a = x;
+#pragma unroll
+  for (int k = 1; k < NB; k++)
+    a = bitsf(__builtin_amdgcn_update_dpp(0, fbits(a), 0x111, 0xf, 0xf, true)) + x;  // row_shr:1
+  return a;
+}
+template <int NB>
+__device__ __forceinline__ float col_spread(float a) {
+  int t = __builtin_amdgcn_update_dpp(0, fbits(a), 0xff, 0xf, 0xf, true);  // each quad's last
+  if constexpr (NB == 8) {
+    t = __builtin_amdgcn_update_dpp(t, t, 0x141, 0xf, 0x5, false);  // lower quads: half row mirrored
+  } else {
+    t = __builtin_amdgcn_update_dpp(t, t, 0x141, 0xf, 0x4, false);
+    t = __builtin_amdgcn_update_dpp(t, t, 0x140, 0xf, 0x3, false);  // lower half: row mirrored
+  }
+  return bitsf(t);
+}
+// The delta rule over the batch's tokens in order: a one-wave workgroup holds 64 / NB columns of one
+// live value head's state, lane c NB + b rows 16 b .. 16 b + 15 of column c (one of ATen's
+// 16-row cascade blocks), NB = 8 blocks where the live key dims end at 128 (the rows past them are
+// zero and stay so), else 16. A token is a serial chain of ~140 vector ops: the block's dot with k, the
+// blocks in order across the column's lanes, the update, the dot with q. No barrier and no
+// LDS: a lane's 16 key and query values come from memory (L2) three tokens ahead, in four fixed
+// buffers. A head's waves go to one XCD, which then holds its queries and keys in its L2. Bound by the
+// chain's issue (148 vector ops a token): 0.49 us a token and layer at 32 live heads of 128 key dims,
+// where 8-wave workgroups of 32 columns, whose sums crossed waves through LDS (three barriers a
+// token), took 1.66. No faster: this token's query dot interleaved with the next one's key dot (0.56),
+// the same with the inputs eight tokens at a time through LDS (0.52).
+struct GdnIn {
+  typedef float v4p __attribute__((ext_vector_type(4), aligned(4)));
+  v4p k[4], q[4];
+  float v, beta, e, lq, lk;
 };
-__global__ __launch_bounds__(NT) void pb_gdn(PbGdn a) {
-  __shared__ PbLds l;
-  const int t = tid(), blk = blockIdx.x;
-  const int nk = a.nk, rl = a.rl, nvr = nk * rl * VD, n = a.n;
-  const int vslot = blk / QC, c0 = (blk % QC) * QW, kh = vslot / rl, vh = kh * a.R + vslot % rl;
-  const int c = t % QW, rb = t / QW;
-  float* S = a.rec + (size_t)vh * KD * VD + c0 + c + rb * 16 * VD;
+template <bool ALL>
+__device__ __forceinline__ float dot16(const float (&s)[16], const GdnIn::v4p (&w)[4]) {
+  float acc = 0.0f;
+#pragma unroll
+  for (int i = 0; i < 16; i++) {
+    const float x = w[i / 4][i % 4], y = acc + s[i] * x;
+    acc = ALL || x != 0.0f ? y : acc;
+  }
+  return acc;
+}
+template <int NB, bool ALL>
+__device__ __forceinline__ float gdn_token(const GdnIn& in, float (&s)[16]) {
+  const float kv = col_spread<NB>(col_last<NB>(dot16<ALL>(s, in.k)));
+  const float d = (in.v - kv) * in.beta;
+#pragma unroll
+  for (int i = 0; i < 16; i++) {
+    const float x = in.k[i / 4][i % 4], y = s[i] + x * d;
+    s[i] = ALL || x != 0.0f ? y : s[i];
+  }
+  return col_last<NB>(dot16<ALL>(s, in.q));
+}
+template <int NB>
+__global__ __launch_bounds__(64) void pb_gdn(PbGdn a) {
+  constexpr int CW = 64 / NB, WS = VD / CW;
+  const int lane = tid(), b = lane % NB, xcd = blockIdx.x & 7, j = blockIdx.x >> 3;
+  const int nk = a.nk, rl = a.rl, nh = nk * rl, nvr = nh * VD, n = a.n;
+  const int vslot = xcd + 8 * (j / WS), col = (j % WS) * CW + lane / NB;
+  if (vslot >= nh) return;
+  const int kh = vslot / rl, vh = kh * a.R + vslot % rl;
+  float* S = a.rec + (size_t)vh * KD * VD + (size_t)(16 * b) * VD + col;
   float s[16];
 #pragma unroll
   for (int i = 0; i < 16; i++) s[i] = S[i * VD];
-  for (int i = t; i < n * 2 * KD; i += NT) {
-    const int b = i / (2 * KD), j = i % (2 * KD);
-    (&l.qk[b][0][0])[j] = a.qk[((int64_t)b * nk + kh) * 2 * KD + j];
-  }
-  for (int i = t; i < n * QW; i += NT) {
-    const int b = i / QW, j = i % QW;
-    l.vb[b][j] = a.v[(int64_t)b * nvr + vslot * VD + c0 + j];
-  }
-  if (t < n) {
-    const float* g = a.g + ((int64_t)t * nk * rl + vslot) * 2;
-    l.bg[t][0] = g[0];
-    l.bg[t][1] = g[1];
+  auto load = [&](int t) {
+    GdnIn in;
+    t = t < n ? t : n - 1;  // (past the end: the last token again, unused)
+    const float* qk = a.qk + ((int64_t)t * nk + kh) * 2 * KD + 16 * b;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      in.k[i] = *reinterpret_cast<const GdnIn::v4p*>(qk + KD + 4 * i);
+      in.q[i] = *reinterpret_cast<const GdnIn::v4p*>(qk + 4 * i);
+    }
+    in.v = a.v[(int64_t)t * nvr + vslot * VD + col];
+    const float* g = a.g + ((int64_t)t * nh + vslot) * 2;
+    in.beta = g[0];
+    in.e = g[1];
     const float* lv = a.live + ((int64_t)t * nk + kh) * 2;
-    l.lv[t] = lv[0] != 0.0f || lv[1] != 0.0f ? 1.0f : 0.0f;
-  }
-  lds_barrier();
-  for (int b = 0; b < n; b++) {
-    const float beta = l.bg[b][0], e = l.bg[b][1];
-    if (e != 1.0f) {
+    in.lq = lv[0];
+    in.lk = lv[1];
+    return in;
+  };
+  const bool whole = a.kl == 16 * NB;
+  auto token = [&](const GdnIn& in, int t) {
+    if (in.e != 1.0f) {
 #pragma unroll
-      for (int i = 0; i < 16; i++) s[i] = s[i] * e;
+      for (int i = 0; i < 16; i++) s[i] = s[i] * in.e;
     }
-    float* o_out = a.o + (int64_t)b * nvr + vslot * VD + c0;
-    if (l.lv[b] != 0.0f) {
-      const float* kr = &l.qk[b][1][rb * 16];
-      const float* qr = &l.qk[b][0][rb * 16];
-      float acc = 0.0f;
-#pragma unroll
-      for (int i = 0; i < 16; i++) acc = kr[i] != 0.0f ? acc + s[i] * kr[i] : acc;
-      l.bsk[rb * QW + c] = acc;
-      lds_barrier();
-      if (t < QW) {
-        float kv = 0.0f;
-#pragma unroll
-        for (int q = 0; q < 16; q++) kv = kv + l.bsk[q * QW + t];
-        l.dl[t] = (l.vb[b][t] - kv) * beta;
-      }
-      lds_barrier();
-      const float d = l.dl[c];
-      float o = 0.0f;
-#pragma unroll
-      for (int i = 0; i < 16; i++) {
-        s[i] = kr[i] != 0.0f ? s[i] + kr[i] * d : s[i];
-        o = qr[i] != 0.0f ? o + s[i] * qr[i] : o;
-      }
-      l.bso[rb * QW + c] = o;
-      lds_barrier();
-      if (t < QW) {
-        float q = 0.0f;
-#pragma unroll
-        for (int j = 0; j < 16; j++) q = q + l.bso[j * QW + t];
-        o_out[t] = bf16r(q);
-      }
-    } else if (t < QW) {
-      o_out[t] = 0.0f;
-    }
+    float o = 0.0f;
+    // (a zero factor adds nothing and leaves its row as it is; a token with none needs no tests)
+    if (whole && in.lq == 2.0f && in.lk == 2.0f) o = gdn_token<NB, true>(in, s);
+    else if (in.lq != 0.0f || in.lk != 0.0f) o = gdn_token<NB, false>(in, s);
+    if (b == NB - 1) a.o[(int64_t)t * nvr + vslot * VD + col] = bf16r(o);
+  };
+  // (a buffer is requested again after its token's last use of it: asked for before, the values
+  // would land in other registers and be copied, each copy waiting for its load)
+  GdnIn n0 = load(0), n1 = load(1), n2 = load(2), n3 = load(3);
+  for (int t = 0; t < n; t += 4) {
+    token(n0, t);
+    n0 = load(t + 4);
+    if (t + 1 < n) token(n1, t + 1);
+    n1 = load(t + 5);
+    if (t + 2 < n) token(n2, t + 2);
+    n2 = load(t + 6);
+    if (t + 3 < n) token(n3, t + 3);
+    n3 = load(t + 7);
   }
 #pragma unroll
   for (int i = 0; i < 16; i++) S[i * VD] = s[i];
@@ -1970,7 +2015,7 @@ static void launch_pb(const uint16_t* W, const uint16_t* W2, int nrows, const ui
   else launch_mm<G, MODE, 2>(W, W2, nrows, X, n, out, ldo, og, st);
 }
 // (G of the hidden rows, live value dims, inter) = (40, 64, 144) or (4, 8, 8). A batch's delta rule
-// runs token by token (pb_gdn on PB-token slices), or chunk by chunk (chunked: lxm_gdn_chunk, the
+// runs token by token (pb_gdn), or chunk by chunk (chunked: lxm_gdn_chunk, the
 // batch a whole number of chunks from the prompt's first token but for the prompt's end).
 template <int GH, int GV, int GI>
 static hipError_t pb_layer(const lxm_dn_params* ph, const lxm_dn_layer& ly, const lxm_dn_pbuf* pb,
@@ -2011,16 +2056,9 @@ static hipError_t pb_layer(const lxm_dn_params* ph, const lxm_dn_layer& ly, cons
       if (e) return (hipError_t)e;
     }
   } else {
-    for (int s = 0; s < n; s += PB) {
-      PbGdn gs = g;
-      gs.n = n - s < PB ? n - s : PB;
-      gs.qk += (int64_t)s * nk * 2 * KD;
-      gs.v += (int64_t)s * nvr;
-      gs.g += (int64_t)s * nk * rl * 2;
-      gs.live += (int64_t)s * nk * 2;
-      gs.o += (int64_t)s * nvr;
-      hipLaunchKernelGGL(pb_gdn, dim3(nk * rl * QC), dim3(NT), 0, st, gs);
-    }
+    const int gs = (nk * rl + 7) / 8 * 8;  // slots a multiple of the XCDs
+    if (kl <= 128) hipLaunchKernelGGL(pb_gdn<8>, dim3(gs * 16), dim3(64), 0, st, g);
+    else hipLaunchKernelGGL(pb_gdn<16>, dim3(gs * 32), dim3(64), 0, st, g);
   }
   hipLaunchKernelGGL(pb_gnorm, dim3(n), dim3(PBT), 0, st, pb->o, pb->P, nproj, 2 * nq + nvr,
                      ly.gnorm, ph->geps, nk * rl, GV, pb->ys, ly.conv, n, nk, kl, rl, R);

@@ -152,6 +152,33 @@ def test_dense_prefill_token_tiles(cuda, n):
     check_prefill(n + 1, 2, seed=3)
 
 
+@pytest.mark.parametrize("kl,zeros", [(128, True), (160, False), (160, True), (256, False)])
+def test_dense_prefill_key_dims(cuda, kl, zeros):
+    """The delta rule's forms: 8 row blocks up to 128 live key dims and 16 beyond; tokens whose query
+    and key hold zeros among the live dims (a third of the query/key rows zero) and a key head that
+    is all zero, beside tokens with none."""
+    from dataclasses import replace
+
+    from oracle import oracle as ox
+
+    spec = replace(synth.config4_small(), kd_live=kl)
+    dm = synth.build_dense(spec, "cpu")
+    conv0, rec0 = synth.dense_state(dm, 3)
+    if zeros:
+        for ly in dm.layers:
+            ly["qk"][:, :, ::3] = 0
+            ly["qk"][:, 1] = 0
+    conv0[:, :2 * spec.nk * 256] = 0.0
+    toks = [int(x) for x in np.random.default_rng(17).integers(0, spec.vocab, 21)]
+    print(f"[gpu-test] dense prefill key dims: kl={kl} zeros={zeros}", flush=True)
+    cache = fast.StateCache(conv0, rec0, "bf16", "cuda")
+    dense.DenseDecode(synth.dense_to(dm, "cuda"), cache).prefill(toks)
+    c, r = conv0.copy(), rec0.copy()
+    ox.OracleModel(synth.to_sparse(dm)).decode(c, r, toks, len(toks))
+    assert (bits(cache.conv_numpy()) == bits(c)).all()
+    assert (bits(cache.rec_numpy()) == bits(r)).all()
+
+
 @pytest.mark.parametrize("chunked,nt", [(0, 16), (0, 48), (1, 64), (1, 128)])
 def test_dense_prefill_batches(cuda, chunked, nt):
     """The C entries with buffers of nt tokens (16 and 64: lxm_dn_prefill and
