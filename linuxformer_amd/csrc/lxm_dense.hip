@@ -1479,6 +1479,7 @@ __global__ __launch_bounds__(PBT, 2) void pb_mm(const uint16_t* __restrict__ W,
   for (int d = 0; d < PD; d++) load(st[(d + 2) % PD]);
   lds_barrier();
   operands(f, 0);
+  lds_barrier();  // (step 0's buffer is read: the first step writes it)
   int par = 0;  // the step's parity: its buffer
   auto sum = [&](v16f (&c)[TN]) {  // one stage's NC steps: this wave's group, from zero
 #pragma unroll

@@ -179,6 +179,25 @@ def test_dense_prefill_key_dims(cuda, kl, zeros):
     assert (bits(cache.rec_numpy()) == bits(r)).all()
 
 
+@pytest.mark.parametrize("n", [5, 40])
+def test_dense_prefill_repeats(cuda, n):
+    """The same prompt twice leaves the same bits at the full row lengths (a short prompt's kernels
+    keep many workgroups a CU, whose waves drift apart: a stage written before every wave has read
+    it shows as a difference between runs)."""
+    spec, dm_cpu, _ = model("mid")
+    dm = synth.dense_to(dm_cpu, "cuda")
+    conv0, rec0 = synth.dense_state(dm_cpu, 3)
+    toks = [int(x) for x in np.random.default_rng(n).integers(0, spec.vocab, n)]
+    print(f"[gpu-test] dense prefill repeats: n={n}", flush=True)
+    out = []
+    for _ in range(6):
+        cache = fast.StateCache(conv0, rec0, "bf16", "cuda")
+        dense.DenseDecode(dm, cache).prefill(toks)
+        out.append((cache.conv_numpy(), cache.rec_numpy()))
+    for a in out[1:]:
+        assert (bits(a[0]) == bits(out[0][0])).all() and (bits(a[1]) == bits(out[0][1])).all()
+
+
 @pytest.mark.parametrize("chunked,nt", [(0, 16), (0, 48), (1, 64), (1, 128)])
 def test_dense_prefill_batches(cuda, chunked, nt):
     """The C entries with buffers of nt tokens (16 and 64: lxm_dn_prefill and
