@@ -43,11 +43,21 @@ typedef struct lxm_chunk_io {
   int32_t o_bf16;  /* 1: o rounded to bf16 (the stock casts the output to the model dtype) */
 } lxm_chunk_io;
 
-/* One chunk of every slot on stream (one workgroup per slot and 32 state columns). q, k, v and S
+/* One chunk of every slot on stream (one workgroup per slot and 16 state columns). q, k, v and S
    are read 16 bytes at a time: each must be 16-byte aligned and qk_ts, qk_hs and v_ts multiples of
    4. Returns a hipError_t (hipErrorInvalidValue for sizes outside the limits above or a misaligned
    pointer or stride). */
 int lxm_gdn_chunk(const lxm_chunk_io* io, void* stream);
+
+/* The chunks of a sequence of T positions (io->n is not read), every slot, in order: what
+   lxm_gdn_chunk on positions 0 .. 63, 64 .. 127, ... leaves, in two launches per group of chunks:
+   what needs no state for the whole group at once, then the chunks in order. ws: a 16-byte aligned
+   device workspace of ws_bytes, at least LXM_CHUNK_WS x n_slots (one chunk a group); with
+   LXM_CHUNK_WS x n_slots x the number of chunks there is one group. Its contents mean nothing
+   between calls. Returns a hipError_t (hipErrorInvalidValue as lxm_gdn_chunk, or for a workspace
+   too small). */
+#define LXM_CHUNK_WS 76304 /* bytes per (slot, chunk) */
+int lxm_gdn_chunks(const lxm_chunk_io* io, int T, void* ws, int64_t ws_bytes, void* stream);
 
 #ifdef __cplusplus
 }

@@ -131,11 +131,13 @@ int lxm_dn_prefill_chunked(const lxm_dn_params* p_host, const int32_t* tokens, i
 
 /* Both prompts with buffers of nt tokens (buf's arrays hold nt tokens each: the sizes above with
    PB = nt): lxm_dn_prefill's results (chunked 0) or lxm_dn_prefill_chunked's (chunked 1; nt a
-   multiple of LXM_CHUNK, buf->gl set), in batches of nt tokens. A batch's rows run on the matrix
+   multiple of LXM_CHUNK, buf->gl set, and past one chunk a workspace ws of ws_bytes as
+   lxm_gdn_chunks takes it for nk x rl slots; else ws may be null), in batches of nt tokens. A batch's rows run on the matrix
    cores at any nt with the same bits; a larger nt reads each weight row fewer times. Returns a
    hipError_t. */
 int lxm_dn_prefill_n(const lxm_dn_params* p_host, const int32_t* tokens, int T,
-                     const lxm_dn_pbuf* buf, int nt, int chunked, void* stream);
+                     const lxm_dn_pbuf* buf, int nt, int chunked, void* ws,
+                     int64_t ws_bytes, void* stream);
 
 #ifdef __cplusplus
 }

@@ -15,6 +15,15 @@ import torch
 from . import mk_build
 
 CHUNK = 64
+CHUNK_WS = 76304       # bytes of workspace per (value head, chunk) (LXM_CHUNK_WS)
+WS_MAX = 160 << 20     # a call's workspace at most (68 chunks of 32 heads; more go in groups)
+
+
+def workspace(n_slots: int, T: int, device) -> torch.Tensor:
+    """The workspace of a T-position call (lxm_gdn_chunks): every chunk's, or what WS_MAX holds."""
+    nch = (T + CHUNK - 1) // CHUNK
+    return torch.empty(n_slots * CHUNK_WS * max(1, min(nch, WS_MAX // (n_slots * CHUNK_WS))),
+                       dtype=torch.uint8, device=device)
 
 
 class ChunkIO(ctypes.Structure):
@@ -38,16 +47,19 @@ def gated_delta_chunked(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: to
     assert nv % nk == 0 and 0 < kl <= 128 and kl % 16 == 0
     for t in (q, k, v, g, beta, S):
         assert t.dtype == torch.float32 and t.is_contiguous() and t.is_cuda
-    o = torch.zeros(T, nv, 128, dtype=torch.float32, device=q.device)
+    o = torch.empty(T, nv, 128, dtype=torch.float32, device=q.device)
+    if T == 0:
+        return o
     st = ctypes.c_void_p(torch.cuda.current_stream(q.device).cuda_stream)
-    for c0 in range(0, T, CHUNK):
-        n = min(CHUNK, T - c0)
-        io = ChunkIO(q=q[c0].data_ptr(), k=k[c0].data_ptr(), v=v[c0].data_ptr(),
-                     beta=beta[c0].data_ptr(), g=g[c0].data_ptr(), S=S.data_ptr(),
-                     o=o[c0].data_ptr(), qk_ts=nk * 256, qk_hs=256, v_ts=nv * 128, g_ts=nv,
-                     g_hs=1, gl_ts=nv, o_ts=nv * 128, n=n, n_slots=nv, rl=nv // nk,
-                     rfull=nv // nk, kl=kl, o_bf16=int(o_bf16))
+    io = ChunkIO(q=q.data_ptr(), k=k.data_ptr(), v=v.data_ptr(), beta=beta.data_ptr(),
+                 g=g.data_ptr(), S=S.data_ptr(), o=o.data_ptr(), qk_ts=nk * 256, qk_hs=256,
+                 v_ts=nv * 128, g_ts=nv, g_hs=1, gl_ts=nv, o_ts=nv * 128, n=min(T, CHUNK),
+                 n_slots=nv, rl=nv // nk, rfull=nv // nk, kl=kl, o_bf16=int(o_bf16))
+    if T <= CHUNK:  # (one launch, no workspace)
         e = lib.lxm_gdn_chunk(ctypes.byref(io), st)
-        if e:
-            raise RuntimeError(f"lxm_gdn_chunk failed: hipError {e}")
+    else:
+        ws = workspace(nv, T, q.device)
+        e = lib.lxm_gdn_chunks(ctypes.byref(io), T, ctypes.c_void_p(ws.data_ptr()), ws.numel(), st)
+    if e:
+        raise RuntimeError(f"lxm_gdn_chunk failed: hipError {e}")
     return o

@@ -1,20 +1,27 @@
 // The stock forward's chunked delta rule (torch_chunk_gated_delta_rule, transformers qwen3_5
-// :249-327) for one chunk of <= 64 positions, on MI355X's matrix cores.
+// :249-327) in chunks of <= 64 positions, on MI355X's matrix cores.
 //
-// One workgroup (8 waves) per (value head, 32 state columns). Everything a chunk needs sits in
-// LDS as fp32 (the keys and queries over the live key dims, the state's 32 columns, the values
-// times beta), and every matrix product is a sequence of v_mfma_f32_16x16x4_f32 (a 16 x 16 tile
-// += 16 x 4 times 4 x 16; lane l supplies A[l % 16][l / 16] and B[l / 16][l % 16] and holds
-// D[4 (l / 16) + r][l % 16], r = 0..3):
-//   A2 = (q k^T) * Gamma,   Gamma[i][j] = exp(gc_i - gc_j) for j <= i, else 0  (gc: cumsum g)
-//   O1 = (q exp(gc)) S
-//   L  = (k beta k^T) * Gamma below the diagonal;  T = (I + L)^-1  (the stock loop's result + I)
-//   W  = T (k beta exp(gc));  U = T (v beta);  v_new = U - W S
-//   o  = O1 + A2 v_new;  S <- S exp(g_last) + (k exp(g_last - gc))^T v_new
-// T is formed by blocks of 16: each diagonal block by forward substitution on one wave, then the
-// blocks below it one block row at a time, T_ij = -T_ii (sum_{k=j}^{i-1} L_ik T_kj), on MFMA.
-// The workgroups of a head repeat the head's Gram matrices and inverse (they are small) and each
-// takes its own 32 columns of the state, so the grid has no dependency between workgroups.
+// Per (value head, chunk), with gc the cumulative sum of g and Gamma[i][j] = exp(gc_i - gc_j) for
+// j <= i, else 0:
+//   A2 = (q k^T) * Gamma;  L = (k beta k^T) * Gamma below the diagonal;  T = (I + L)^-1  (the
+//   stock loop's result + I);  W = T (k beta exp(gc));  U = T (v beta)
+//   v_new = U - W S;  o = (q exp(gc)) S + A2 v_new;  S <- S exp(g_last) + (k exp(g_last - gc))^T v_new
+// A2, W and U need no state, so a sequence's chunks form them in parallel (chunk_prep, one
+// workgroup per (head, chunk), into a workspace); what is left of a chunk is a short chain in the
+// state (chunk_run, one workgroup per (head, 16 state columns), its chunks in order, the state
+// in registers and LDS). One chunk alone (chunk_one) does both in one launch with no workspace.
+//
+// Every product is v_mfma_f32_16x16x4_f32 (a 16 x 16 tile += 16 x 4 times 4 x 16; lane l supplies
+// A[l % 16][l / 16] and B[l / 16][l % 16] and holds D[4 (l / 16) + r][l % 16], r = 0..3), its k
+// ascending, so each result is one chain of fused multiply-adds in k order whatever the kernel.
+// Operands come as 16 bytes a lane (a block of 16 k: lane group g's k = g, 4 + g, 8 + g, 12 + g):
+// rows lie in LDS with each block of 16 transposed as 4 x 4 (pos16), tiles in LDS and in the
+// workspace as operands, a D tile turned into a B operand by four 4-byte LDS writes a lane.
+//
+// A chunk's chain is bound by its latency: a wave's two products of 32 MFMAs, a barrier, a triangular one
+// and one of 32, a barrier, where one workgroup per (head, chunk, 32 columns)
+// and a launch a chunk took 31 us, each column block repeating the inverse. 2,048 positions of 32 heads:
+// 1,020 -> 234 us (chunk_prep 68, chunk_run 179: 5.6 a chunk); 100 positions of 4 heads 62.3 -> 34.4.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -25,322 +32,586 @@ using namespace lxm;
 
 namespace {
 
-constexpr int CT = 512;       // threads per workgroup (8 waves: two per SIMD)
-constexpr int NWV = CT / 64;
-constexpr int C = 64;         // positions per chunk
-constexpr int KL = 128;       // live key dims at most
+constexpr int CT = 256;  // threads per workgroup (4 waves: one per 16 positions)
+constexpr int C = LXM_CHUNK;
+constexpr int KL = 128;  // live key dims at most
 constexpr int VD = 128;
-constexpr int VT = 32;        // state columns per workgroup
-constexpr int SK = KL + 4;    // row strides in floats (LDS padding)
-constexpr int SC = C + 4;
-constexpr int SV = VT + 4;
-constexpr int ST = 16 + 1;
-
-struct ChunkLds {
-  float k[C][SK];             // keys (rows past n and dims past kl: 0)
-  float qw[C][SK];            // queries, then W = T (k beta exp(gc))
-  float a2[C][SC];            // (q k^T) * Gamma
-  float lp[C][SC];            // L = (k beta k^T) * Gamma, strictly lower; later v_new
-  float tt[C][SC];            // T = (I + L)^-1
-  float s[KL][SV];            // the state's columns
-  float vb[C][SV];            // v beta
-  float pt[4][16][ST];        // per-wave 16 x 16 scratch (the block inverse)
-  float gc[C], eg[C], f[C], beta[C];
-  float misc[4];
-};
-static_assert(sizeof(ChunkLds) <= 160 * 1024, "one workgroup's LDS");
+constexpr int VT = 16;       // state columns per workgroup
+constexpr int SK = KL + 4;   // row strides in floats: of rows read along k (16 rows on 16 bank groups),
+constexpr int SR = KL + 16;  // of rows read across (4 rows x 16 columns on 64 banks),
+constexpr int SC = C + 4;    // of the 64 x 64 matrices
+constexpr int NTRI = 10;     // 16 x 16 tiles on or below the diagonal
+// a (head, chunk)'s workspace in floats: W's 32 tiles and A2's 10 as A operands, U's 32 as D tiles,
+// then eg, f and el
+constexpr int WS_A2 = 32 * 256, WS_U = WS_A2 + NTRI * 256, WS_V = WS_U + 32 * 256;
 
 typedef float v4f __attribute__((ext_vector_type(4)));
 
-__device__ __forceinline__ v4f mfma4(float a, float b, v4f c) {
-  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+struct Vecs {
+  float gc[C], beta[C], eg[C], f[C];  // (f = exp(g_last - gc))
+  float el[4];                        // exp(g_last)
+};
+struct StepLds {  // B operands: the state's tiles and v_new
+  v4f s[KL / 16][64], vn[4][64];
+};
+struct PrepLds {
+  union {
+    float kq[2][C][SK];  // k and q (blocks transposed), read by the Gram products; in their place
+    struct {
+      float kb[C][SR];   // k beta exp(gc), then v beta
+      float lp[C][SC], tt[C][SC];
+    };
+  };
+  v4f pt[4][64];         // per-wave scratch
+  Vecs v;
+};
+struct RunLds {
+  float k[C][SR], q[C][SK];
+  StepLds st;
+};
+struct OneLds {
+  float q[C][SK];
+  union {
+    float k[C][SK];
+    float kb[C][SR];     // after the Gram products: k beta exp(gc), then k
+  };
+  union {
+    float lp[C][SC];
+    float w[C][SK];      // W (blocks transposed) once L is read
+  };
+  float tt[C][SC], a2[C][SC];
+  v4f pt[4][64];
+  Vecs v;
+  StepLds st;
+};
+static_assert(2 * sizeof(PrepLds) <= 160 * 1024 && sizeof(OneLds) <= 160 * 1024, "LDS");
+static_assert(LXM_CHUNK_WS == 4 * (WS_V + 2 * C + 4), "workspace");
+
+__device__ __forceinline__ v4f mfma4(const v4f& a, const v4f& b, v4f c) {
+#pragma unroll
+  for (int r = 0; r < 4; r++) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[r], b[r], c, 0, 0, 0);
+  return c;
+}
+// A chain of MFMAs that ends inside a branch is waited for there: where the branch's end joined
+// another path, the compiler has read the last MFMA's rows with no wait states in between (the last
+// row of the tile came out without its last four terms).
+__device__ __forceinline__ void settle(v4f& c) { asm volatile("s_nop 15" : "+v"(c)); }
+__device__ __forceinline__ v4f ld4(const float* p) { return *reinterpret_cast<const v4f*>(p); }
+__device__ __forceinline__ void st4(float* p, const v4f& v) { *reinterpret_cast<v4f*>(p) = v; }
+__device__ __forceinline__ int wave() { return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); }
+// what this wave's lanes stored in LDS, for its other lanes (a wave's LDS accesses run in order)
+__device__ __forceinline__ void wave_sync() {
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+  __builtin_amdgcn_wave_barrier();
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+}
+__device__ __forceinline__ int tri(int ti, int tj) { return ti * (ti + 1) / 2 + tj; }
+__device__ __forceinline__ void tri_of(int p, int& ti, int& tj) {
+  ti = p < 1 ? 0 : p < 3 ? 1 : p < 6 ? 2 : 3;
+  tj = p - ti * (ti + 1) / 2;
+}
+// column c of a row whose blocks of 16 are transposed as 4 x 4: lane group g's four k of a block
+// are 16 consecutive bytes
+__device__ __forceinline__ int pos16(int c) { return (c & ~15) | ((c & 3) << 2) | ((c >> 2) & 3); }
+__device__ __forceinline__ void st_pos16(float* row, int d, const v4f& v) {  // d a multiple of 4
+  float* p = row + (d & ~15) + ((d >> 2) & 3);
+#pragma unroll
+  for (int c = 0; c < 4; c++) p[4 * c] = v[c];
+}
+// element (i, j) of a tile as A operand: its float in the tile's 256
+__device__ __forceinline__ int a_pos(int i, int j) {
+  return ((i & 15) + 16 * (j & 3)) * 4 + ((j >> 2) & 3);
+}
+// a D tile as B operand into dst[64]
+__device__ __forceinline__ void st_b(v4f* dst, const v4f& d) {
+  const int lane = threadIdx.x & 63, i16 = lane & 15, g = lane >> 4;
+  float* p = reinterpret_cast<float*>(dst) + i16 * 4 + g;
+#pragma unroll
+  for (int r = 0; r < 4; r++) p[64 * r] = d[r];
+}
+// the block of 16 k from k0 of column c of rows of stride S, as B operand
+template <int S>
+__device__ __forceinline__ v4f ld_b(const float* m, int k0, int c) {
+  const int g = (threadIdx.x & 63) >> 4;
+  v4f b;
+#pragma unroll
+  for (int r = 0; r < 4; r++) b[r] = m[(k0 + 4 * r + g) * S + c];
+  return b;
+}
+// the block of 16 k from k0 of row i of rows of stride SC, as A operand
+__device__ __forceinline__ v4f ld_a(const float* m, int i, int k0) {
+  const int g = (threadIdx.x & 63) >> 4;
+  v4f a;
+#pragma unroll
+  for (int r = 0; r < 4; r++) a[r] = m[i * SC + k0 + 4 * r + g];
+  return a;
 }
 
-// the tile's lane coordinates: A/B operand row (or column) a_i and k index a_k; D rows d_i + r
-struct Lane {
-  int a_i, a_k, d_i, d_j;
-  __device__ Lane() {
-    const int l = threadIdx.x & 63;
-    a_i = l & 15;
-    a_k = l >> 4;
-    d_i = 4 * (l >> 4);
-    d_j = l & 15;
+// A chunk's n positions from p0, thread t: rows t / 32 + 8 j, dims 4 (t % 32) (below kl; rows past
+// n: zero)
+__device__ __forceinline__ void load_rows(const float* m, int64_t ts, int64_t off, int n,
+                                          v4f (&x)[C / 8]) {
+  const int d = 4 * (threadIdx.x & 31);
+#pragma unroll
+  for (int j = 0; j < C / 8; j++) {
+    const int i = (threadIdx.x >> 5) + 8 * j, ic = i < n ? i : n - 1;
+    x[j] = ld4(m + off + ic * ts + d);
   }
-};
+#pragma unroll
+  for (int j = 0; j < C / 8; j++) {
+    const v4f z = {0.0f, 0.0f, 0.0f, 0.0f};
+    x[j] = (int)(threadIdx.x >> 5) + 8 * j < n ? x[j] : z;
+  }
+}
+// rows (row(i), dims 4 (t % 32)) from x
+template <class F>
+__device__ __forceinline__ void each_row(F f) {
+#pragma unroll
+  for (int j = 0; j < C / 8; j++) f((int)(threadIdx.x >> 5) + 8 * j, 4 * (int)(threadIdx.x & 31), j);
+}
 
-__device__ __forceinline__ int wave() { return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); }
+// A2 and T of head h's chunk of n positions from p0, whose keys kv (load_rows) the caller holds. k,
+// q: LDS rows of SK (blocks transposed); between() is called once they are read (by every wave) and
+// before lp and tt are written; a2(i, j, x) stores A2[i][j] (tiles on or below the diagonal). After
+// it every wave may read v, tt, and what between and a2 stored in LDS.
+template <class FB, class FA>
+__device__ __forceinline__ void prep(const lxm_chunk_io& io, int h, int64_t p0, int n,
+                                     const v4f (&kv)[C / 8], float* k, float* q, float* lp,
+                                     float* tt, v4f* pt, Vecs& v, FB between, FA a2) {
+  const int t = threadIdx.x, w = wave(), lane = t & 63, i16 = lane & 15, g = lane >> 4;
+  const int kl = io.kl;
+  {
+    v4f qv[C / 8];
+    if (4 * (t & 31) < kl) {
+      load_rows(io.q, io.qk_ts, p0 * io.qk_ts + (int64_t)(h / io.rl) * io.qk_hs, n, qv);
+      each_row([&](int i, int d, int j) {
+        st_pos16(k + i * SK, d, kv[j]);
+        st_pos16(q + i * SK, d, qv[j]);
+      });
+    }
+  }
+  if (w == 0) {  // the vectors: position = lane. gc: binary64 sums in order, each prefix rounded
+    float b = 0.0f, gr = 0.0f;
+    if (lane < n) {
+      b = io.beta[(p0 + lane) * io.g_ts + (int64_t)h * io.g_hs];
+      gr = io.g[(p0 + lane) * io.gl_ts + h];
+    }
+    double a = 0.0;
+    float gc = 0.0f;
+#pragma unroll
+    for (int i = 0; i < C; i++) {
+      a += (double)__uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(gr), i));
+      gc = lane == i ? (float)a : gc;
+    }
+    const float gl = (float)a;
+    v.gc[lane] = gc;
+    v.beta[lane] = b;
+    v.eg[lane] = cr_exp(gc);
+    v.f[lane] = cr_exp(gl - gc);
+    if (lane == 0) v.el[0] = cr_exp(gl);
+  }
+  lds_barrier();
+  // ---- the Gram tiles, dealt to the waves
+  v4f aq[3], ak[3];
+#pragma unroll
+  for (int u = 0; u < 3; u++) {
+    aq[u] = ak[u] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    const int p = w + 4 * u;
+    if (p >= NTRI) continue;
+    int ti, tj;
+    tri_of(p, ti, tj);
+    const float bi = v.beta[16 * ti + i16];
+    const float *qi = q + (16 * ti + i16) * SK + 4 * g, *ki = k + (16 * ti + i16) * SK + 4 * g,
+                *kj = k + (16 * tj + i16) * SK + 4 * g;
+    v4f a = ld4(qi), b = ld4(ki), c = ld4(kj);
+    for (int d0 = 0; d0 < kl; d0 += 16) {
+      const int dn = d0 + 16 < kl ? d0 + 16 : d0;  // (the last block again, unused)
+      const v4f an = ld4(qi + dn), bn = ld4(ki + dn), cn = ld4(kj + dn);
+      aq[u] = mfma4(a, c, aq[u]);
+      ak[u] = mfma4(b * bi, c, ak[u]);
+      a = an;
+      b = bn;
+      c = cn;
+    }
+    settle(aq[u]);
+    settle(ak[u]);
+  }
+  lds_barrier();
+  between();
+#pragma unroll
+  for (int u = 0; u < 3; u++) {
+    const int p = w + 4 * u;
+    if (p >= NTRI) continue;
+    int ti, tj;
+    tri_of(p, ti, tj);
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int i = 16 * ti + 4 * g + r, j = 16 * tj + i16;
+      const float gm = j <= i ? cr_exp(v.gc[i] - v.gc[j]) : 0.0f;
+      a2(i, j, aq[u][r] * gm);
+      lp[i * SC + j] = j < i ? ak[u][r] * gm : 0.0f;
+    }
+  }
+  lds_barrier();
+  // ---- T: diagonal block w by forward substitution, lane % 16 its column in registers
+  {
+    const float* lb = lp + 16 * w * SC + 16 * w;
+    float tc[16];
+    tc[0] = i16 == 0 ? 1.0f : 0.0f;
+#pragma unroll
+    for (int i = 1; i < 16; i++) {
+      float s = 0.0f;
+#pragma unroll
+      for (int m4 = 0; m4 < (i + 3) / 4; m4++) {
+        const v4f l4 = ld4(lb + i * SC + 4 * m4);
+#pragma unroll
+        for (int m = 0; m < 4; m++)
+          if (4 * m4 + m < i) s = s + l4[m] * tc[4 * m4 + m];
+      }
+      tc[i] = i16 < i ? -s : i16 == i ? 1.0f : 0.0f;
+    }
+    if (lane < 16) {
+#pragma unroll
+      for (int i = 0; i < 16; i++) tt[(16 * w + i) * SC + 16 * w + i16] = tc[i];
+    }
+  }
+  lds_barrier();
+  // block rows 1..3: T_ij = -T_ii P, P = sum_{m=j}^{i-1} L_im T_mj; block (i, j) on wave j
+  for (int bi = 1; bi < 4; bi++) {
+    if (w < bi) {
+      const v4f z = {0.0f, 0.0f, 0.0f, 0.0f};
+      v4f p = z;
+      for (int m = w; m < bi; m++)
+        p = mfma4(ld_a(lp, 16 * bi + i16, 16 * m), ld_b<SC>(tt, 16 * m, 16 * w + i16), p);
+      settle(p);
+      st_b(pt + 64 * w, p);
+      wave_sync();
+      v4f x = mfma4(ld_a(tt, 16 * bi + i16, 16 * bi), pt[64 * w + lane], z);
+      settle(x);
+#pragma unroll
+      for (int r = 0; r < 4; r++) tt[(16 * bi + 4 * g + r) * SC + 16 * w + i16] = -x[r];
+    }
+    lds_barrier();
+  }
+}
+// tile (ti, column block at c) of T times rows of stride SR (T is lower triangular: k blocks <= ti)
+__device__ __forceinline__ v4f t_times(const float* tt, const float* m, int ti, int c) {
+  const int i16 = threadIdx.x & 15;
+  v4f a = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int kb = 0; kb < 4; kb++)
+    if (kb <= ti) a = mfma4(ld_a(tt, 16 * ti + i16, 16 * kb), ld_b<SR>(m, 16 * kb, c + i16), a);
+  return a;
+}
 
-// acc += A B over k blocks kb0 .. kb1 - 1 of 16 (k = 16 kb + 4 j + a_k): fa(k) and fb(k) give
-// this lane's A and B elements. Each block's 8 operands are read before the previous block's 4
-// MFMAs issue, so the LDS reads overlap the matrix core.
-template <class FA, class FB>
-__device__ __forceinline__ v4f tile_mm(int kb0, int kb1, const Lane& ln, FA fa, FB fb, v4f acc) {
-  if (kb0 >= kb1) return acc;
-  float a[4], b[4];
+// One chunk's step for 16 state columns: wave w holds positions 16 w .. 16 w + 15 and state tiles
+// 2 w and 2 w + 1 (s; every tile in st.s as B operand). wa, qa, aa(t): the wave's rows of W, q
+// exp(gc) and A2 as A operands; u: U's tile; k: the chunk's keys, rows of SR in LDS; f[t][r] of
+// position 16 t + 4 r + g. mid(): after W, q and U are read. Returns o's tile; the new state in s and
+// st.s (behind a barrier of the caller's).
+template <class WA, class QA, class AA, class Mid>
+__device__ __forceinline__ v4f chunk_step(StepLds& st, const float* k, int nkt, WA wa, QA qa,
+                                          const v4f& u, const v4f (&f)[4], float el, AA aa,
+                                          v4f (&s)[2], Mid mid) {
+  const int w = wave(), lane = threadIdx.x & 63, i16 = lane & 15;
+  const v4f z = {0.0f, 0.0f, 0.0f, 0.0f};
+  v4f vp = z, o1 = z;
 #pragma unroll
-  for (int j = 0; j < 4; j++) {
-    a[j] = fa(16 * kb0 + 4 * j + ln.a_k);
-    b[j] = fb(16 * kb0 + 4 * j + ln.a_k);
+  for (int t = 0; t < KL / 16; t++) {  // (zeros past kl)
+    const v4f b = st.s[t][lane];
+    vp = mfma4(wa(t), b, vp);
+    o1 = mfma4(qa(t), b, o1);
   }
-  for (int kb = kb0; kb < kb1; kb++) {
-    float an[4], bn[4];
-    const int kn = kb + 1 < kb1 ? kb + 1 : kb;  // (the last block reads its own operands again)
+  st_b(st.vn[w], u - vp);
+  mid();
+  lds_barrier();
+  v4f b[4], x[2] = {z, z};
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-      an[j] = fa(16 * kn + 4 * j + ln.a_k);
-      bn[j] = fb(16 * kn + 4 * j + ln.a_k);
+  for (int t = 0; t < 4; t++) b[t] = st.vn[t][lane];
+  v4f a = mfma4(aa(0), b[0], z);
+  if (w > 0) {
+    a = mfma4(aa(1), b[1], a);
+    if (w > 1) {
+      a = mfma4(aa(2), b[2], a);
+      if (w > 2) a = mfma4(aa(3), b[3], a);
+      settle(a);
     }
-#pragma unroll
-    for (int j = 0; j < 4; j++) acc = mfma4(a[j], b[j], acc);
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-      a[j] = an[j];
-      b[j] = bn[j];
-    }
+    settle(a);
   }
-  return acc;
+#pragma unroll
+  for (int t = 0; t < 4; t++)
+#pragma unroll
+    for (int j = 0; j < 2; j++)
+      x[j] = mfma4(ld_b<SR>(k, 16 * t, 16 * (2 * w + j) + i16) * f[t], b[t], x[j]);
+#pragma unroll
+  for (int j = 0; j < 2; j++) {
+    x[j] = s[j] * el + x[j];
+    s[j] = 2 * w + j < nkt ? x[j] : z;
+    st_b(st.s[2 * w + j], s[j]);
+  }
+  return o1 + a;
+}
+
+__device__ __forceinline__ float* state_of(const lxm_chunk_io& io, int h, int c0) {
+  return io.S + ((size_t)(h / io.rl) * io.rfull + h % io.rl) * 256 * VD + c0;
+}
+__device__ __forceinline__ void load_state(const float* S, int nkt, StepLds& st, v4f (&s)[2]) {
+  const int w = wave(), lane = threadIdx.x & 63, i16 = lane & 15, g = lane >> 4;
+#pragma unroll
+  for (int j = 0; j < 2; j++) {
+    s[j] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    if (2 * w + j < nkt) {
+#pragma unroll
+      for (int r = 0; r < 4; r++) s[j][r] = S[(size_t)(16 * (2 * w + j) + 4 * g + r) * VD + i16];
+    }
+    st_b(st.s[2 * w + j], s[j]);
+  }
+}
+__device__ __forceinline__ void store_state(float* S, int nkt, const v4f (&s)[2]) {
+  const int w = wave(), lane = threadIdx.x & 63, i16 = lane & 15, g = lane >> 4;
+#pragma unroll
+  for (int j = 0; j < 2; j++)
+    if (2 * w + j < nkt) {
+#pragma unroll
+      for (int r = 0; r < 4; r++) S[(size_t)(16 * (2 * w + j) + 4 * g + r) * VD + i16] = s[j][r];
+    }
+}
+__device__ __forceinline__ void store_o(const lxm_chunk_io& io, int h, int c0, int64_t p0, int n,
+                                        const v4f& o) {
+  const int w = wave(), lane = threadIdx.x & 63, i16 = lane & 15, g = lane >> 4;
+#pragma unroll
+  for (int r = 0; r < 4; r++) {
+    const int i = 16 * w + 4 * g + r;
+    if (i < n)
+      io.o[(p0 + i) * io.o_ts + (int64_t)h * VD + c0 + i16] = io.o_bf16 ? bf16r(o[r]) : o[r];
+  }
+}
+// (workgroups are dealt to the 8 XCDs in turn: a head's 8 column groups on one of them, whose L2
+// then holds its keys, queries, T and A2)
+__device__ __forceinline__ bool head_cols(int n_slots, int& h, int& c0) {
+  const int x = blockIdx.x & 7, j = blockIdx.x >> 3;
+  h = x + 8 * (j / (VD / VT));
+  c0 = (j % (VD / VT)) * VT;
+  return h < n_slots;
 }
 
 }  // namespace
 
-__global__ __launch_bounds__(CT) void lxm_chunk_k(lxm_chunk_io io) {
+// W, U, A2 and the vectors of every (head, chunk), chunks ch0 .. ch0 + gridDim.y - 1 of T positions
+__global__ __launch_bounds__(CT, 2) void chunk_prep(lxm_chunk_io io, int T, int ch0, float* ws) {
   extern __shared__ __align__(16) uint8_t smem_raw[];
-  ChunkLds& l = *reinterpret_cast<ChunkLds*>(smem_raw);
-  const int t = threadIdx.x, w = wave(), h = blockIdx.x, c0 = blockIdx.y * VT;
-  const int n = io.n, kl = io.kl, kh = h / io.rl;
-  const Lane ln;
-  float* Sg = io.S + ((size_t)kh * io.rfull + h % io.rl) * 256 * VD;
-  constexpr int NKB = KL / 16;  // k blocks over the key dims (zeros past kl add nothing)
+  PrepLds& l = *reinterpret_cast<PrepLds*>(smem_raw);
+  const int h = blockIdx.x, ch = ch0 + blockIdx.y, n = T - ch * C < C ? T - ch * C : C;
+  const int w = wave(), lane = threadIdx.x & 63, i16 = lane & 15, g = lane >> 4;
+  const int64_t p0 = (int64_t)ch * C;
+  const bool mine = 4 * (int)(threadIdx.x & 31) < io.kl;
+  float* o = ws + ((size_t)blockIdx.y * io.n_slots + h) * (LXM_CHUNK_WS / 4);
+  v4f kv[C / 8], vv[C / 8];
+  if (mine) load_rows(io.k, io.qk_ts, p0 * io.qk_ts + (int64_t)(h / io.rl) * io.qk_hs, n, kv);
+  prep(io, h, p0, n, kv, &l.kq[0][0][0], &l.kq[1][0][0], &l.lp[0][0], &l.tt[0][0], &l.pt[0][0], l.v,
+       [&] {
+         if (mine)
+           each_row([&](int i, int d, int j) {
+             st4(&l.kb[i][d], (kv[j] * l.v.beta[i]) * l.v.eg[i]);
+           });
+         load_rows(io.v, io.v_ts, p0 * io.v_ts + (int64_t)h * VD, n, vv);
+       },
+       [&](int i, int j, float x) { o[WS_A2 + tri(i >> 4, j >> 4) * 256 + a_pos(i, j)] = x; });
+  // wave w: the column blocks w and w + 4 of W, then of U
+  for (int tc = w; 16 * tc < io.kl; tc += 4)
+#pragma unroll
+    for (int ti = 0; ti < 4; ti++) {
+      const v4f a = t_times(&l.tt[0][0], &l.kb[0][0], ti, 16 * tc);
+#pragma unroll
+      for (int r = 0; r < 4; r++) o[(ti * 8 + tc) * 256 + a_pos(4 * g + r, i16)] = a[r];
+    }
+  lds_barrier();  // (kb is read)
+  each_row([&](int i, int d, int j) { st4(&l.kb[i][d], vv[j] * l.v.beta[i]); });
+  lds_barrier();
+  for (int tc = w; tc < VD / 16; tc += 4)
+#pragma unroll
+    for (int ti = 0; ti < 4; ti++)
+      st4(o + WS_U + (ti * 8 + tc) * 256 + 4 * lane, t_times(&l.tt[0][0], &l.kb[0][0], ti, 16 * tc));
+  if (threadIdx.x < C) {
+    o[WS_V + threadIdx.x] = l.v.eg[threadIdx.x];
+    o[WS_V + C + threadIdx.x] = l.v.f[threadIdx.x];
+    if (threadIdx.x == 0) o[WS_V + 2 * C] = l.v.el[0];
+  }
+}
 
-  // ---- inputs into LDS (zero past n positions and kl dims), four values per load
-  for (int idx = t; idx < C * KL / 4; idx += CT) {
-    const int i = idx / (KL / 4), d = 4 * (idx % (KL / 4));
-    v4f kv = {0.0f, 0.0f, 0.0f, 0.0f}, qv = kv;
-    if (i < n && d < kl) {
-      const int64_t o = (int64_t)i * io.qk_ts + (int64_t)kh * io.qk_hs + d;
-      kv = *reinterpret_cast<const v4f*>(io.k + o);
-      qv = *reinterpret_cast<const v4f*>(io.q + o);
+// the chunks ch0 .. ch0 + nch - 1 in order for 16 state columns of a head; each operand is
+// requested for the next chunk right after its last use
+__global__ __launch_bounds__(CT, 1) void chunk_run(lxm_chunk_io io, int T, int ch0, int nch,
+                                                   const float* ws) {
+  __shared__ RunLds l;
+  int h, c0;
+  if (!head_cols(io.n_slots, h, c0)) return;
+  const int w = wave(), lane = threadIdx.x & 63, i16 = lane & 15, g = lane >> 4;
+  const int nkt = io.kl / 16, kh = h / io.rl, row = 16 * w + i16;
+  float* S = state_of(io, h, c0);
+  v4f s[2], wa[KL / 16], ka[KL / 16], qa[KL / 16], ar[4], f[4], u;
+  float eg, el;
+  auto wsc = [&](int c) { return ws + ((size_t)c * io.n_slots + h) * (LXM_CHUNK_WS / 4); };
+  auto get_kq = [&](int c) {  // (positions past the end: the last, taken as zero below)
+    const int p = (ch0 + c) * C + row;
+    const int64_t o = (int64_t)(p < T ? p : T - 1) * io.qk_ts + (int64_t)kh * io.qk_hs + 4 * g;
+    const float* x = wsc(c);
+#pragma unroll
+    for (int t = 0; t < KL / 16; t++) {  // (blocks past kl: the last one's, taken as zero)
+      const int tk = t < nkt ? t : nkt - 1;
+      ka[t] = ld4(io.k + o + 16 * tk);
+      qa[t] = ld4(io.q + o + 16 * tk);
+      wa[t] = ld4(x + (w * 8 + tk) * 256 + 4 * lane);
     }
-    *reinterpret_cast<v4f*>(&l.k[i][d]) = kv;
-    *reinterpret_cast<v4f*>(&l.qw[i][d]) = qv;
-  }
-  if (t < C) {
-    float b = 0.0f, g = 0.0f;
-    if (t < n) {
-      b = io.beta[(int64_t)t * io.g_ts + (int64_t)h * io.g_hs];
-      g = io.g[(int64_t)t * io.gl_ts + h];
+    eg = x[WS_V + row];
+    u = ld4(x + WS_U + (w * 8 + c0 / 16) * 256 + 4 * lane);
+  };
+  auto get_rest = [&](int c) {
+    const float* x = wsc(c);
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+      if (t <= w) ar[t] = ld4(x + WS_A2 + tri(w, t) * 256 + 4 * lane);
+#pragma unroll
+      for (int r = 0; r < 4; r++) f[t][r] = x[WS_V + C + 16 * t + 4 * r + g];
     }
-    l.beta[t] = b;
-    l.gc[t] = g;
-  }
-  for (int idx = t; idx < KL * VT / 4; idx += CT) {
-    const int d = idx / (VT / 4), c = 4 * (idx % (VT / 4));
-    v4f sv = {0.0f, 0.0f, 0.0f, 0.0f};
-    if (d < kl) sv = *reinterpret_cast<const v4f*>(Sg + (size_t)d * VD + c0 + c);
-    *reinterpret_cast<v4f*>(&l.s[d][c]) = sv;
-  }
-  __syncthreads();
-  if (t == 0) {  // cumsum of g: binary64 accumulation, each prefix rounded (ATen's CPU cumsum)
-    double acc = 0.0;
-    for (int i = 0; i < C; i++) {
-      acc += (double)l.gc[i];
-      l.gc[i] = (float)acc;
+    el = x[WS_V + 2 * C];
+  };
+  load_state(S, nkt, l.st, s);
+  get_kq(0);
+  get_rest(0);
+  lds_barrier();
+  for (int c = 0; c < nch; c++) {
+    const int p0 = (ch0 + c) * C, n = T - p0 < C ? T - p0 : C;
+    const int cn = c + 1 < nch ? c + 1 : c;  // (the last chunk's again, unused)
+    const v4f z = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int t = 0; t < KL / 16; t++) {
+      const bool in = row < n && t < nkt;
+      st4(&l.k[row][16 * t + 4 * g], in ? ka[t] : z);
+      st_pos16(l.q[row], 16 * t + 4 * g, in ? qa[t] * eg : z);
+      wa[t] = t < nkt ? wa[t] : z;
     }
+    wave_sync();  // (a wave reads its own rows of q)
+    const v4f o = chunk_step(
+        l.st, &l.k[0][0], nkt, [&](int t) { return wa[t]; },
+        [&](int t) { return ld4(&l.q[row][16 * t + 4 * g]); }, u, f, el,
+        [&](int t) { return ar[t]; }, s, [&] { get_kq(cn); });
+    store_o(io, h, c0, p0, n, o);
+    get_rest(cn);
+    lds_barrier();  // (the state's tiles for every wave; k and v_new are read)
   }
-  for (int idx = t; idx < C * VT / 4; idx += CT) {
-    const int i = idx / (VT / 4), c = 4 * (idx % (VT / 4));
-    v4f vv = {0.0f, 0.0f, 0.0f, 0.0f};
-    if (i < n) vv = *reinterpret_cast<const v4f*>(io.v + (int64_t)i * io.v_ts + (int64_t)h * VD + c0 + c);
-    const float b = l.beta[i];
-    *reinterpret_cast<v4f*>(&l.vb[i][c]) = v4f{vv.x * b, vv.y * b, vv.z * b, vv.w * b};
-  }
-  __syncthreads();
-  if (t < C) {
-    const float glast = l.gc[C - 1];
-    l.eg[t] = cr_exp(l.gc[t]);
-    l.f[t] = cr_exp(glast - l.gc[t]);
-    if (t == 0) l.misc[0] = cr_exp(glast);
-  }
-  __syncthreads();
+  store_state(S, nkt, s);
+}
 
-  // ---- A2 = (q k^T) * Gamma and L = (k beta k^T) * Gamma (strictly lower) on the 10 tiles on
-  // or below the diagonal, dealt to the waves (tile p: row block ti, column block tj <= ti);
-  // O1 = (q exp(gc)) S: wave w takes row block w % 4, column tile w / 4
-  for (int p = w; p < 10; p += NWV) {
-    const int ti = p < 1 ? 0 : p < 3 ? 1 : p < 6 ? 2 : 3;
-    const int tj = p - ti * (ti + 1) / 2;
-    const int ia = 16 * ti + ln.a_i, jb = 16 * tj + ln.a_i;
-    const float bi = l.beta[ia];
-    v4f aq = {0.0f, 0.0f, 0.0f, 0.0f}, ak = aq;
-    float qa[4], ka[4], kb[4];
+// one chunk of every head: A2, T and W repeated by each of a head's 8 workgroups, each with its own
+// columns of U
+__global__ __launch_bounds__(CT, 1) void chunk_one(lxm_chunk_io io) {
+  extern __shared__ __align__(16) uint8_t smem_raw[];
+  OneLds& l = *reinterpret_cast<OneLds*>(smem_raw);
+  int h, c0;
+  if (!head_cols(io.n_slots, h, c0)) return;
+  const int w = wave(), lane = threadIdx.x & 63, i16 = lane & 15, g = lane >> 4;
+  const int nkt = io.kl / 16, n = io.n, row = 16 * w + i16;
+  const bool mine = 4 * (int)(threadIdx.x & 31) < io.kl;
+  float* S = state_of(io, h, c0);
+  v4f kv[C / 8], s[2], vb[4], f[4];
+  if (mine) {
+    load_rows(io.k, io.qk_ts, (int64_t)(h / io.rl) * io.qk_hs, n, kv);
+  } else {  // (dims past kl: zero in every product)
+    const v4f z = {0.0f, 0.0f, 0.0f, 0.0f};
+    each_row([&](int i, int d, int j) {
+      kv[j] = z;
+      st4(&l.q[i][d], z);
+    });
+  }
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-      qa[j] = l.qw[ia][4 * j + ln.a_k];
-      ka[j] = l.k[ia][4 * j + ln.a_k] * bi;
-      kb[j] = l.k[jb][4 * j + ln.a_k];
-    }
-    for (int d0 = 0; d0 < KL; d0 += 16) {
-      float qn[4], kn[4], bn[4];
-      const int dn = d0 + 16 < KL ? d0 + 16 : d0;
-#pragma unroll
-      for (int j = 0; j < 4; j++) {
-        qn[j] = l.qw[ia][dn + 4 * j + ln.a_k];
-        kn[j] = l.k[ia][dn + 4 * j + ln.a_k] * bi;
-        bn[j] = l.k[jb][dn + 4 * j + ln.a_k];
-      }
-#pragma unroll
-      for (int j = 0; j < 4; j++) {
-        aq = mfma4(qa[j], kb[j], aq);
-        ak = mfma4(ka[j], kb[j], ak);
-      }
-#pragma unroll
-      for (int j = 0; j < 4; j++) {
-        qa[j] = qn[j];
-        ka[j] = kn[j];
-        kb[j] = bn[j];
-      }
-    }
+  for (int t = 0; t < 4; t++)  // v's 16 columns as B operand
 #pragma unroll
     for (int r = 0; r < 4; r++) {
-      const int i = 16 * ti + ln.d_i + r, j = 16 * tj + ln.d_j;
-      const float gm = j <= i ? cr_exp(l.gc[i] - l.gc[j]) : 0.0f;
-      l.a2[i][j] = aq[r] * gm;
-      l.lp[i][j] = j < i ? ak[r] * gm : 0.0f;
+      const int i = 16 * t + 4 * r + g;
+      vb[t][r] = i < n ? io.v[i * io.v_ts + (int64_t)h * VD + c0 + i16] : 0.0f;
     }
-  }
-  // the six tiles above the diagonal are zero in both
-  for (int idx = t; idx < 6 * 256; idx += CT) {
-    const int p = idx / 256, e = idx % 256;
-    const int ti = p < 3 ? 0 : p < 5 ? 1 : 2, tj = p < 3 ? p + 1 : p < 5 ? p - 1 : 3;
-    l.a2[16 * ti + e / 16][16 * tj + e % 16] = 0.0f;
-    l.lp[16 * ti + e / 16][16 * tj + e % 16] = 0.0f;
-  }
-  const int ob = w & 3, oc = w >> 2;  // this wave's output tile of the (64, 32) products
-  v4f o1 = {0.0f, 0.0f, 0.0f, 0.0f};
-  {
-    const int ia = 16 * ob + ln.a_i;
-    const float e = l.eg[ia];
-    o1 = tile_mm(0, NKB, ln, [&](int k) { return l.qw[ia][k] * e; },
-                 [&](int k) { return l.s[k][16 * oc + ln.a_i]; }, o1);
-  }
-  __syncthreads();
-
-  // ---- T = (I + L)^-1: diagonal block w (waves 0..3) by forward substitution (lanes 0..15
-  // are the columns: T[i][j] = -sum_{m=j}^{i-1} L[i][m] T[m][j], T[i][i] = 1); blocks above
-  // the diagonal are zero
-  if (w < 4) {
-    const int b0 = 16 * w, j = t & 63;
-    if (j < 16) l.tt[b0][b0 + j] = j == 0 ? 1.0f : 0.0f;
-    __builtin_amdgcn_wave_barrier();
-    for (int i = 1; i < 16; i++) {
-      if (j < 16) {
-        float s = 0.0f;
-        for (int m = j; m < i; m++) s = s + l.lp[b0 + i][b0 + m] * l.tt[b0 + m][b0 + j];
-        l.tt[b0 + i][b0 + j] = j < i ? -s : (j == i ? 1.0f : 0.0f);
-      }
-      __builtin_amdgcn_wave_barrier();
+  load_state(S, nkt, l.st, s);
+  prep(io, h, 0, n, kv, &l.k[0][0], &l.q[0][0], &l.lp[0][0], &l.tt[0][0], &l.pt[0][0], l.v,
+       [&] {
+         each_row([&](int i, int d, int j) {
+           st4(&l.kb[i][d], (kv[j] * l.v.beta[i]) * l.v.eg[i]);
+         });
+       },
+       [&](int i, int j, float x) { l.a2[i][j] = x; });
+#pragma unroll 1
+  for (int tc = w; tc < KL / 16; tc += 4)
+#pragma unroll
+    for (int ti = 0; ti < 4; ti++) {
+      const v4f a = t_times(&l.tt[0][0], &l.kb[0][0], ti, 16 * tc);
+#pragma unroll
+      for (int r = 0; r < 4; r++) l.w[16 * ti + 4 * g + r][pos16(16 * tc + i16)] = a[r];
     }
-  } else {
-    for (int idx = t - 256; idx < 6 * 256; idx += 256) {
-      const int p = idx / 256, e = idx % 256;
-      const int ti = p < 3 ? 0 : p < 5 ? 1 : 2, tj = p < 3 ? p + 1 : p < 5 ? p - 1 : 3;
-      l.tt[16 * ti + e / 16][16 * tj + e % 16] = 0.0f;
-    }
-  }
-  __syncthreads();
-  // block rows 1..3: T_ij = -T_ii P, P = sum_{k=j}^{i-1} L_ik T_kj; block (i, j) on wave j
-  for (int bi = 1; bi < 4; bi++) {
-    if (w < bi) {
-      const int bj = w;
-      v4f p = {0.0f, 0.0f, 0.0f, 0.0f};
-      p = tile_mm(bj, bi, ln, [&](int k) { return l.lp[16 * bi + ln.a_i][k]; },
-                  [&](int k) { return l.tt[k][16 * bj + ln.a_i]; }, p);
+  v4f u = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-      for (int r = 0; r < 4; r++) l.pt[w][ln.d_i + r][ln.d_j] = p[r];
-      __builtin_amdgcn_wave_barrier();
-      v4f q = {0.0f, 0.0f, 0.0f, 0.0f};
-      q = tile_mm(0, 1, ln, [&](int k) { return l.tt[16 * bi + ln.a_i][16 * bi + k]; },
-                  [&](int k) { return l.pt[w][k][ln.a_i]; }, q);
-#pragma unroll
-      for (int r = 0; r < 4; r++) l.tt[16 * bi + ln.d_i + r][16 * bj + ln.d_j] = -q[r];
-    }
-    __syncthreads();
-  }
-
-  // ---- W = T (k beta exp(gc)) into qw (the queries are no longer read): the 32 tiles (4 row
-  // blocks x 8 column blocks) dealt to the waves; T is lower triangular (k blocks <= the row's)
-  for (int p = w; p < 32; p += NWV) {
-    const int ti = p & 3, tc = p >> 2;
-    v4f a = {0.0f, 0.0f, 0.0f, 0.0f};
-    a = tile_mm(0, ti + 1, ln, [&](int k) { return l.tt[16 * ti + ln.a_i][k]; },
-                [&](int k) { return (l.k[k][16 * tc + ln.a_i] * l.beta[k]) * l.eg[k]; }, a);
-#pragma unroll
-    for (int r = 0; r < 4; r++) l.qw[16 * ti + ln.d_i + r][16 * tc + ln.d_j] = a[r];
-  }
-  __syncthreads();
-
-  // ---- v_new = T (v beta) - W S on the wave's output tile, into lp (L was last read by the
-  // block stages, before the barriers above)
-  {
-    v4f u = {0.0f, 0.0f, 0.0f, 0.0f}, vp = u;
-    u = tile_mm(0, ob + 1, ln, [&](int k) { return l.tt[16 * ob + ln.a_i][k]; },
-                [&](int k) { return l.vb[k][16 * oc + ln.a_i]; }, u);
-    vp = tile_mm(0, NKB, ln, [&](int k) { return l.qw[16 * ob + ln.a_i][k]; },
-                 [&](int k) { return l.s[k][16 * oc + ln.a_i]; }, vp);
-#pragma unroll
-    for (int r = 0; r < 4; r++) l.lp[16 * ob + ln.d_i + r][16 * oc + ln.d_j] = u[r] - vp[r];
-  }
-  __syncthreads();
-
-  // ---- o = O1 + A2 v_new on the wave's output tile (A2 is lower triangular)
-  {
-    v4f a = {0.0f, 0.0f, 0.0f, 0.0f};
-    a = tile_mm(0, ob + 1, ln, [&](int k) { return l.a2[16 * ob + ln.a_i][k]; },
-                [&](int k) { return l.lp[k][16 * oc + ln.a_i]; }, a);
+  for (int t = 0; t < 4; t++) {
+    v4f b;
 #pragma unroll
     for (int r = 0; r < 4; r++) {
-      const int i = 16 * ob + ln.d_i + r, c = 16 * oc + ln.d_j;
-      if (i < n) {
-        const float v = o1[r] + a[r];
-        io.o[(int64_t)i * io.o_ts + (int64_t)h * VD + c0 + c] = io.o_bf16 ? bf16r(v) : v;
-      }
+      const int i = 16 * t + 4 * r + g;
+      b[r] = vb[t][r] * l.v.beta[i];
+      f[t][r] = l.v.f[i];
+    }
+    if (t <= w) {
+      u = mfma4(ld_a(&l.tt[0][0], row, 16 * t), b, u);
+      settle(u);
     }
   }
-  // ---- S <- S exp(g_last) + (k f)^T v_new: the state's 16 tiles (8 row blocks x 2 column
-  // tiles) dealt to the waves (row blocks past kl skipped)
-  {
-    const float el = l.misc[0];
-    for (int p = w; p < 2 * KL / 16; p += NWV) {
-      const int rb = p >> 1, tc = p & 1;
-      if (16 * rb >= kl) continue;
-      v4f a = {0.0f, 0.0f, 0.0f, 0.0f};
-      a = tile_mm(0, C / 16, ln, [&](int m) { return l.k[m][16 * rb + ln.a_i] * l.f[m]; },
-                  [&](int m) { return l.lp[m][16 * tc + ln.a_i]; }, a);
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const int d = 16 * rb + ln.d_i + r, c = 16 * tc + ln.d_j;
-        Sg[(size_t)d * VD + c0 + c] = l.s[d][c] * el + a[r];
-      }
-    }
-  }
+  lds_barrier();  // (kb is read: the keys in its place, behind the step's barrier)
+  each_row([&](int i, int d, int j) { st4(&l.kb[i][d], kv[j]); });
+  const float eg = l.v.eg[row];
+  const v4f o = chunk_step(
+      l.st, &l.kb[0][0], nkt, [&](int t) { return ld4(&l.w[row][16 * t + 4 * g]); },
+      [&](int t) { return ld4(&l.q[row][16 * t + 4 * g]) * eg; }, u, f, l.v.el[0],
+      [&](int t) { return ld_a(&l.a2[0][0], row, 16 * t); }, s, [] {});
+  store_o(io, h, c0, 0, n, o);
+  store_state(S, nkt, s);
 }
 
 // q, k, v and S are read four floats at a time: their pointers 16-byte aligned, and the strides
 // between those reads multiples of 4 floats
 static bool al16(const void* p) { return ((uintptr_t)p & 15) == 0; }
+static bool io_ok(const lxm_chunk_io* io) {
+  return io && io->kl >= 1 && io->kl <= KL && io->kl % 16 == 0 && io->n_slots >= 1 && io->rl >= 1 &&
+         io->rfull >= io->rl && al16(io->q) && al16(io->k) && al16(io->v) && al16(io->S) &&
+         io->qk_ts % 4 == 0 && io->qk_hs % 4 == 0 && io->v_ts % 4 == 0;
+}
+static int cols_grid(int n_slots) { return (n_slots + 7) / 8 * 8 * (VD / VT); }
 
 extern "C" int lxm_gdn_chunk(const lxm_chunk_io* io, void* stream) {
-  if (!io || io->n < 1 || io->n > C || io->kl < 1 || io->kl > KL || io->kl % 16 != 0 ||
-      io->n_slots < 1 || io->rl < 1 || io->rfull < io->rl)
-    return (int)hipErrorInvalidValue;
-  if (!al16(io->q) || !al16(io->k) || !al16(io->v) || !al16(io->S) || io->qk_ts % 4 != 0 ||
-      io->qk_hs % 4 != 0 || io->v_ts % 4 != 0)
-    return (int)hipErrorInvalidValue;
-  const int lds = (int)sizeof(ChunkLds);
-  hipError_t e = hipFuncSetAttribute((const void*)lxm_chunk_k,
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  if (!io_ok(io) || io->n < 1 || io->n > C) return (int)hipErrorInvalidValue;
+  const int lds = (int)sizeof(OneLds);
+  const hipError_t e = hipFuncSetAttribute((const void*)chunk_one,
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, lds);
   if (e != hipSuccess) return (int)e;
-  hipLaunchKernelGGL(lxm_chunk_k, dim3(io->n_slots, VD / VT), dim3(CT), lds,
-                     (hipStream_t)stream, *io);
+  hipLaunchKernelGGL(chunk_one, dim3(cols_grid(io->n_slots)), dim3(CT), lds, (hipStream_t)stream,
+                     *io);
+  return (int)hipGetLastError();
+}
+
+extern "C" int lxm_gdn_chunks(const lxm_chunk_io* io, int T, void* ws, int64_t ws_bytes,
+                              void* stream) {
+  if (!io_ok(io) || T < 1 || !al16(ws)) return (int)hipErrorInvalidValue;
+  const int64_t per = (int64_t)LXM_CHUNK_WS * io->n_slots;
+  const int nch = (int)(((int64_t)T + C - 1) / C);
+  int64_t grp = ws ? ws_bytes / per : 0;  // chunks the workspace holds
+  if (grp < 1) return (int)hipErrorInvalidValue;
+  if (grp > 65535) grp = 65535;  // (a grid's y extent)
+  const int lds = (int)sizeof(PrepLds);
+  const hipError_t e = hipFuncSetAttribute((const void*)chunk_prep,
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  if (e != hipSuccess) return (int)e;
+  for (int c = 0; c < nch; c += (int)grp) {
+    const int m = nch - c < grp ? nch - c : (int)grp;
+    hipLaunchKernelGGL(chunk_prep, dim3(io->n_slots, m), dim3(CT), lds, (hipStream_t)stream, *io, T, c,
+                       static_cast<float*>(ws));
+    hipLaunchKernelGGL(chunk_run, dim3(cols_grid(io->n_slots)), dim3(CT), 0, (hipStream_t)stream,
+                       *io, T, c, m, static_cast<const float*>(ws));
+  }
   return (int)hipGetLastError();
 }

@@ -2016,11 +2016,11 @@ static void launch_pb(const uint16_t* W, const uint16_t* W2, int nrows, const ui
   else launch_mm<G, MODE, 2>(W, W2, nrows, X, n, out, ldo, og, st);
 }
 // (G of the hidden rows, live value dims, inter) = (40, 64, 144) or (4, 8, 8). A batch's delta rule
-// runs token by token (pb_gdn), or chunk by chunk (chunked: lxm_gdn_chunk, the
+// runs token by token (pb_gdn), or chunk by chunk (chunked: lxm_gdn_chunks, the
 // batch a whole number of chunks from the prompt's first token but for the prompt's end).
 template <int GH, int GV, int GI>
 static hipError_t pb_layer(const lxm_dn_params* ph, const lxm_dn_layer& ly, const lxm_dn_pbuf* pb,
-                           int n, bool chunked, hipStream_t st) {
+                           int n, bool chunked, void* ws, int64_t ws_bytes, hipStream_t st) {
   const int H = ph->hidden, I = ph->inter, nk = ph->nk, kl = ph->kl, rl = ph->rl, R = ph->nv / nk;
   const int nq = nk * kl, nvr = nk * rl * VD, nproj = 2 * nq + 2 * nvr + 2 * nk * rl;
   const float eps = ph->rms_eps;
@@ -2045,17 +2045,15 @@ static hipError_t pb_layer(const lxm_dn_params* ph, const lxm_dn_layer& ly, cons
     io.rfull = R;
     io.kl = kl;
     io.o_bf16 = 1;
-    for (int s = 0; s < n; s += LXM_CHUNK) {
-      io.q = pb->qk + s * io.qk_ts;
-      io.k = io.q + KD;
-      io.v = pb->v + s * io.v_ts;
-      io.beta = pb->g + s * io.g_ts;
-      io.g = pb->gl + s * io.gl_ts;
-      io.o = pb->o + s * io.o_ts;
-      io.n = n - s < LXM_CHUNK ? n - s : LXM_CHUNK;
-      const int e = lxm_gdn_chunk(&io, st);
-      if (e) return (hipError_t)e;
-    }
+    io.q = pb->qk;
+    io.k = pb->qk + KD;
+    io.v = pb->v;
+    io.beta = pb->g;
+    io.g = pb->gl;
+    io.o = pb->o;
+    io.n = n;
+    const int e = n <= LXM_CHUNK ? lxm_gdn_chunk(&io, st) : lxm_gdn_chunks(&io, n, ws, ws_bytes, st);
+    if (e) return (hipError_t)e;
   } else {
     const int gs = (nk * rl + 7) / 8 * 8;  // slots a multiple of the XCDs
     if (kl <= 128) hipLaunchKernelGGL(pb_gdn<8>, dim3(gs * 16), dim3(64), 0, st, g);
@@ -2071,9 +2069,11 @@ static hipError_t pb_layer(const lxm_dn_params* ph, const lxm_dn_layer& ly, cons
 }
 
 extern "C" int lxm_dn_prefill_n(const lxm_dn_params* ph, const int32_t* tokens, int T,
-                                const lxm_dn_pbuf* pb, int nt, int chunked, void* stream) {
+                                const lxm_dn_pbuf* pb, int nt, int chunked, void* ws, int64_t ws_bytes,
+                                void* stream) {
   if (!dims_ok(ph) || !pb || !tokens || T < 0 || nt < 1) return (int)hipErrorInvalidValue;
-  if (chunked && (!pb->gl || ph->kl > 128 || ph->kl % 16 || nt % LXM_CHUNK))
+  if (chunked && (!pb->gl || ph->kl > 128 || ph->kl % 16 || nt % LXM_CHUNK ||
+                  (nt > LXM_CHUNK && (!ws || ws_bytes < (int64_t)LXM_CHUNK_WS * ph->nk * ph->rl))))
     return (int)hipErrorInvalidValue;
   const int gh = g_of(ph->hidden), gv = g_of(ph->nk * ph->rl * VD), gi = g_of(ph->inter);
   const bool full = gh == 40 && gv == 64 && gi == 144, small = gh == 4 && gv == 8 && gi == 8;
@@ -2085,8 +2085,8 @@ extern "C" int lxm_dn_prefill_n(const lxm_dn_params* ph, const int32_t* tokens, 
                        ph->vocab, pb->h, ph->err);
     for (int L = 0; L < ph->n_layers; L++) {
       const lxm_dn_layer& ly = ph->layers_host[L];
-      const hipError_t e = full ? pb_layer<40, 64, 144>(ph, ly, pb, n, chunked != 0, st)
-                                : pb_layer<4, 8, 8>(ph, ly, pb, n, chunked != 0, st);
+      const hipError_t e = full ? pb_layer<40, 64, 144>(ph, ly, pb, n, chunked != 0, ws, ws_bytes, st)
+                                : pb_layer<4, 8, 8>(ph, ly, pb, n, chunked != 0, ws, ws_bytes, st);
       if (e != hipSuccess) return (int)e;
     }
   }
@@ -2095,7 +2095,7 @@ extern "C" int lxm_dn_prefill_n(const lxm_dn_params* ph, const int32_t* tokens, 
 
 extern "C" int lxm_dn_prefill(const lxm_dn_params* ph, const int32_t* tokens, int T,
                               const lxm_dn_pbuf* pb, void* stream) {
-  return lxm_dn_prefill_n(ph, tokens, T, pb, PB, 0, stream);
+  return lxm_dn_prefill_n(ph, tokens, T, pb, PB, 0, nullptr, 0, stream);
 }
 
 // The stock forward's prompt (the T > 1 path: Qwen3_5GatedDeltaNet.forward :517-529 calls
@@ -2103,5 +2103,5 @@ extern "C" int lxm_dn_prefill(const lxm_dn_params* ph, const int32_t* tokens, in
 // and states are the chunked form's.
 extern "C" int lxm_dn_prefill_chunked(const lxm_dn_params* ph, const int32_t* tokens, int T,
                                       const lxm_dn_pbuf* pb, void* stream) {
-  return lxm_dn_prefill_n(ph, tokens, T, pb, LXM_CHUNK, 1, stream);
+  return lxm_dn_prefill_n(ph, tokens, T, pb, LXM_CHUNK, 1, nullptr, 0, stream);
 }

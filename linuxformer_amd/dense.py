@@ -22,6 +22,7 @@ import ctypes
 import torch
 
 from . import mk_build
+from .chunk import workspace
 
 P64 = ctypes.c_void_p
 
@@ -178,8 +179,12 @@ class DenseDecode:
         self.err.zero_()
         p, _ = self._params(1)
         st = ctypes.c_void_p(torch.cuda.current_stream(self.dev).cuda_stream)
-        e = self.lib.lxm_dn_prefill_n(ctypes.byref(p), ctypes.c_void_p(tok.data_ptr()),
-                                      int(t.numel()), ctypes.byref(pb), nt, int(chunked), st)
+        T = int(t.numel())
+        ws = workspace(self.spec.nk * self.spec.r_live, min(T, nt), self.dev) if chunked else None
+        e = self.lib.lxm_dn_prefill_n(ctypes.byref(p), ctypes.c_void_p(tok.data_ptr()), T,
+                                      ctypes.byref(pb), nt, int(chunked),
+                                      ctypes.c_void_p(ws.data_ptr() if chunked else None),
+                                      ws.numel() if chunked else 0, st)
         if e:
             raise RuntimeError(f"dense prefill launch failed: hipError {e}")
         torch.cuda.synchronize(self.dev)

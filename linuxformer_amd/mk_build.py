@@ -116,10 +116,12 @@ def load(subprof: bool = False) -> ctypes.CDLL:
         lib.lxm_dn_prefill.restype = I
         lib.lxm_dn_prefill_chunked.argtypes = [P, P, I, P, P]
         lib.lxm_dn_prefill_chunked.restype = I
-        lib.lxm_dn_prefill_n.argtypes = [P, P, I, P, I, I, P]
+        lib.lxm_dn_prefill_n.argtypes = [P, P, I, P, I, I, P, ctypes.c_int64, P]
         lib.lxm_dn_prefill_n.restype = I
         lib.lxm_gdn_chunk.argtypes = [P, P]
         lib.lxm_gdn_chunk.restype = I
+        lib.lxm_gdn_chunks.argtypes = [P, I, P, ctypes.c_int64, P]
+        lib.lxm_gdn_chunks.restype = I
         lib.lxm_t_sync.argtypes = [I, I, I, I, P, P, P, P]
         lib.lxm_t_sync.restype = I
         _libs[path] = lib
@@ -130,4 +132,4 @@ EXPORTS = ("lxm_run", "lxm_lds_base", "lxm_helper_lds", "lxm_max_blocks", "lxm_m
            "lxm_last_error", "lxm_device_cus", "lxm_t_elem", "lxm_t_sum", "lxm_pf_layers",
            "lxm_pf_head", "lxm_pf_embed", "lxm_pf_tiles", "lxm_pf_lds", "lxm_dn_step", "lxm_dn_run",
            "lxm_dn_prefill", "lxm_t_sync", "lxm_run_noalloc", "lxm_gdn_chunk",
-           "lxm_dn_prefill_chunked", "lxm_dn_prefill_n")
+           "lxm_dn_prefill_chunked", "lxm_dn_prefill_n", "lxm_gdn_chunks")

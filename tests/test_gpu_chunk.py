@@ -88,3 +88,36 @@ def test_chunk_exact_regime_bit_exact(cuda, T):
     assert (o == o_ref).all()
     assert (Sg == S_ref).all()
     assert np.abs(o_ref).max() > 0
+
+
+@pytest.mark.parametrize("T,nk,R,kl,groups", [(65, 1, 1, 128, 1), (200, 3, 2, 112, 2),
+                                              (320, 2, 1, 16, 5), (129, 9, 1, 64, 1)])
+def test_chunks_equal_single_chunks(cuda, T, nk, R, kl, groups):
+    """A sequence's chunks at once (lxm_gdn_chunks: what needs no state in parallel, then the chunks in
+    order; in groups of chunks when the workspace is smaller) leave the bits of one lxm_gdn_chunk call
+    per chunk: ragged last chunks of one and eight positions, few key dims, odd head counts."""
+    import ctypes
+
+    from linuxformer_amd import chunk
+
+    print(f"[gpu-test] chunks T={T} nk={nk} R={R} kl={kl} groups={groups}", flush=True)
+    q, k, v, g, beta, S = (torch.from_numpy(a).to(cuda) for a in _inputs(T, nk, R, 11))
+    q[..., kl:] = 0
+    k[..., kl:] = 0
+    S[:, kl:] = 0
+    S1, S2, nv = S.clone(), S.clone(), nk * R
+    parts = [gated_delta_chunked(*(t[i:i + 64].contiguous() for t in (q, k, v, g, beta)), S1, kl=kl)
+             for i in range(0, T, 64)]
+    o = torch.empty(T, nv, 128, device=cuda)
+    io = chunk.ChunkIO(q=q.data_ptr(), k=k.data_ptr(), v=v.data_ptr(), beta=beta.data_ptr(),
+                       g=g.data_ptr(), S=S2.data_ptr(), o=o.data_ptr(), qk_ts=nk * 256, qk_hs=256,
+                       v_ts=nv * 128, g_ts=nv, g_hs=1, gl_ts=nv, o_ts=nv * 128, n=64, n_slots=nv,
+                       rl=R, rfull=R, kl=kl, o_bf16=0)
+    ws = chunk.workspace(nv, 64 * (-(-T // 64) // groups), cuda)
+    lib = mk_build.load()
+    e = lib.lxm_gdn_chunks(ctypes.byref(io), T, ctypes.c_void_p(ws.data_ptr()), ws.numel(), None)
+    assert e == 0
+    torch.cuda.synchronize()
+    assert torch.equal(torch.cat(parts), o) and torch.equal(S1, S2)
+    assert lib.lxm_gdn_chunks(ctypes.byref(io), T, ctypes.c_void_p(ws.data_ptr()),
+                              chunk.CHUNK_WS * nv - 1, None) != 0  # (a workspace too small)

@@ -11,7 +11,7 @@ import numpy as np
 import pytest
 import torch
 
-from linuxformer_amd import dense, fast, mk_build, synth
+from linuxformer_amd import chunk, dense, fast, mk_build, synth
 
 pytestmark = pytest.mark.gpu
 
@@ -227,7 +227,9 @@ def test_dense_prefill_batches(cuda, chunked, nt):
             elif nt == 64:
                 e = dd.lib.lxm_dn_prefill_chunked(*args, st)
             else:
-                e = dd.lib.lxm_dn_prefill_n(*args, nt, chunked, st)
+                ws = chunk.workspace(spec.nk * spec.r_live, 64, "cuda")  # (one chunk a group)
+                e = dd.lib.lxm_dn_prefill_n(*args, nt, chunked, ctypes.c_void_p(ws.data_ptr()),
+                                            ws.numel(), st)
             assert e == 0
             torch.cuda.synchronize()
         out.append((cache.conv_numpy(), cache.rec_numpy()))
