@@ -1370,13 +1370,13 @@ __device__ __forceinline__ uint16_t bf16_bits(float v) { return (uint16_t)(fbits
 // seven regimes of magnitude), and bf16 x bf16 products are exact in fp32: a group's chain of MFMAs
 // from zero is its sum, bit for bit, for 32 rows x 32 tokens at once.
 //
-// A workgroup (4 waves) takes 32 rows x 32 TN tokens. Its waves split the groups, not the tile: wave
+// A workgroup (4 waves) takes 32 rows x 64 tokens. Its waves split the groups, not the tile: wave
 // w takes the groups congruent to w mod 4, so one step stages 4 consecutive groups' chunk q (64
 // bytes of each row and token) and every wave works on its own group of it. The 16 stages run in the
 // tree's order (m bit-reversed), so a wave's tree over its 16 groups is a binary counter of at
 // most 4 pending tiles; the last two levels join the 4 classes through LDS: (c0 + c2) + (c1 + c3).
 //
-// The bound is the fp32 matrix rate. A step is 4 (TN = 1) or 8 MFMAs of 64 cycles a wave; the loads
+// The bound is the fp32 matrix rate. A step is 8 MFMAs of 64 cycles a wave; the loads
 // run PD + 2 steps ahead (PD of them in registers), the LDS buffers 2 steps, a wave's operands 1
 // step; two workgroups share a CU and cover each other's tree and barriers. Per layer of the
 // 2,560 / 4,096 / 9,216 stack at 2,048 tokens: SwiGLU 1.88 ms (103 TFLOP/s), projections 1.24, down_proj
@@ -1391,14 +1391,14 @@ __device__ __forceinline__ uint16_t bf16_bits(float v) { return (uint16_t)(fbits
 // 2 (SwiGLU, a tile's first half of rows from W, the second the same units from W2):
 // out[b ldo + il(u, og)] = D(D(silu(D(g))) * D(u)) (bf16).
 typedef float v16f __attribute__((ext_vector_type(16)));
-template <int G, int MODE, int TN>
+template <int G, int MODE>
 __global__ __launch_bounds__(PBT, 2) void pb_mm(const uint16_t* __restrict__ W,
                                                 const uint16_t* __restrict__ W2, int nrows,
                                                 const uint16_t* __restrict__ X, int n, void* out,
                                                 int ldo, int og, int ntt) {
   constexpr int CH = G == 4 ? 4 : 8, NC = G / CH, K = 64 * G;
   constexpr int PD = NC % 5 == 0 ? 5 : NC % 4 == 0 ? 4 : NC % 3 == 0 ? 3 : 1;  // loads' lead
-  constexpr int RT = 32, TT = 32 * TN, RU = MODE == 2 ? RT / 2 : RT;
+  constexpr int TN = 2, RT = 32, TT = 32 * TN, RU = MODE == 2 ? RT / 2 : RT;
   constexpr int LN = RT + TT, TH = PBT, UN = 4 * LN, UPT = (UN + TH - 1) / TH;
   constexpr int CS = LN + 4;      // a class's stride in 16-byte units (4 classes on 4 bank quarters)
   constexpr int RS = RT + 4;      // the reduction's token stride in floats
@@ -1570,6 +1570,170 @@ __global__ __launch_bounds__(PBT, 2) void pb_mm(const uint16_t* __restrict__ W,
             else o[k] = bf16r(o[k] + bf16r(v[k]));
           }
       }
+    }
+  }
+}
+
+// The same rows and order for up to 64 tokens, where the weights' stream bounds a batch and pb_mm's 32
+// rows a workgroup leave CUs idle (80 workgroups for 2,560 rows): 16 rows x 16 TN tokens on 8
+// waves, v_mfma_f32_16x16x4_f32 (its four k in order, as pb_mm's two). A step stages QS chunks of 8
+// consecutive groups (128 bytes, a whole line, of each row and token); wave w works on group w of the
+// 8, its 8 stages in the tree's order, and the last three levels join the 8 classes through LDS.
+// The loads run PD + 1 steps ahead. A 13-token batch's four products of a layer of the 2,560 / 4,096 /
+// 9,216 stack: 94 us, the vector form 101,
+// pb_mm on 32-token tiles 159 (the weights at 5 TB/s: 45).
+template <int G, int MODE, int TN>
+__global__ __launch_bounds__(NT) void pb_ms(const uint16_t* __restrict__ W,
+                                            const uint16_t* __restrict__ W2, int nrows,
+                                            const uint16_t* __restrict__ X, int n, void* out,
+                                            int ldo, int og) {
+  constexpr int CH = G == 4 ? 4 : 8, NC = G / CH, K = 64 * G;
+  constexpr int QS = TN <= 2 ? (NC % 6 == 0 ? 6 : NC % 5 == 0 ? 5 : NC % 4 == 0 ? 4 : 1)
+                             : (NC % 3 == 0 ? 3 : NC % 2 == 0 ? 2 : 1);
+  constexpr int SP = NC / QS;  // steps of a stage
+  constexpr int PD = SP % 5 == 0 ? 5 : SP % 3 == 0 ? 3 : SP % 2 == 0 ? 2 : 1;
+  constexpr int RT = 16, TT = 16 * TN, RU = MODE == 2 ? RT / 2 : RT;
+  constexpr int LN = RT + TT, UC = 8 * LN, UN = UC * QS, UPT = (UN + NT - 1) / NT;
+  constexpr int CS = LN + 2;   // a class's stride in 16-byte units (8 classes on 8 bank groups)
+  constexpr int RS = RT + 4;   // the reduction's token stride in floats
+  constexpr int BUF = QS * 8 * CS, STG = 2 * BUF * 16, RED = 8 * TT * RS * 4;
+  static_assert(NC % QS == 0 && SP % PD == 0, "a stage's loop is unrolled by the lead");
+  __shared__ __align__(16) uint8_t sm[STG > RED ? STG : RED];
+  v4u* ring = reinterpret_cast<v4u*>(sm);
+  const int r0 = blockIdx.x * RU, t = tid(), lane = t & 63, cls = wave_id();
+  const int i16 = lane & 15, g = lane >> 4;
+  const uint16_t* src[UPT];
+  int dst[UPT];
+#pragma unroll
+  for (int i = 0; i < UPT; i++) {
+    const int u = t + i * NT, qq = u / UC, ln = u % UC / 8, c = u & 7;
+    const uint16_t* base = X;
+    if (ln < RT) {
+      int r = r0 + (MODE == 2 ? ln % RU : ln);
+      r = r < nrows ? r : nrows - 1;  // (rows and tokens past the end: the last one's, unused)
+      base = (MODE == 2 && ln >= RU ? W2 : W) + (int64_t)r * K;
+    } else {
+      base = X + (int64_t)(ln - RT < n ? ln - RT : n - 1) * K;
+    }
+    src[i] = base + (qq * 64 + c) * CH;
+    dst[i] = (qq * 8 + c) * CS + ln;
+  }
+  const bool last = UN % NT == 0 || t + (UPT - 1) * NT < UN;  // (whole waves)
+  v4u st[PD][UPT];
+  int lq = 0, lst = 0;  // the next step to load: its first chunk, its stage
+  auto load = [&](v4u (&s)[UPT]) {
+    const int m = ((lst & 1) << 2) | (lst & 2) | ((lst & 4) >> 2);
+    const int off = (lq * 64 + 8 * m) * CH;
+#pragma unroll
+    for (int i = 0; i < UPT; i++) {
+      if (i + 1 < UPT || last) {
+        if constexpr (CH == 8) {
+          s[i] = *reinterpret_cast<const v4u*>(src[i] + off);
+        } else {
+          const uint2 v = *reinterpret_cast<const uint2*>(src[i] + off);
+          s[i] = v4u{v.x, v.y, 0u, 0u};
+        }
+      }
+    }
+    lq += QS;
+    if (lq == NC) {  // (past the last step: the last stage again, unused)
+      lq = 0;
+      lst = lst < 7 ? lst + 1 : 7;
+    }
+  };
+  auto stage = [&](const v4u (&s)[UPT], int p) {
+#pragma unroll
+    for (int i = 0; i < UPT; i++)
+      if (i + 1 < UPT || last) ring[p * BUF + dst[i]] = s[i];
+  };
+  // lane group g holds k = g (of a chunk's first four) and 4 + g: halves of words g / 2, 2 + g / 2
+  const uint32_t sel = g & 1 ? 0x07060c0cu : 0x05040c0cu;
+  auto val = [&](uint32_t w) { return bitsf(__builtin_amdgcn_perm(w, 0u, sel)); };
+  v4f acc[TN], p0[TN], p1[TN], p2[TN];
+#pragma unroll
+  for (int i = 0; i < TN; i++) p0[i] = p1[i] = p2[i] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+  v4u s0[UPT];
+  load(s0);
+#pragma unroll
+  for (int d = 0; d < PD; d++) load(st[(d + 1) % PD]);
+  stage(s0, 0);
+  lds_barrier();
+  int par = 0;  // the step's parity: its buffer
+#pragma unroll 1
+  for (int sg = 0; sg < 8; sg++) {
+#pragma unroll
+    for (int i = 0; i < TN; i++) acc[i] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int d = 0; d < SP; d++) {
+      // the next step into the other buffer (read before the last barrier); this step's products
+      stage(st[(d + 1) % PD], par ^ 1);
+      load(st[(d + 1) % PD]);
+      const uint32_t* b = reinterpret_cast<const uint32_t*>(ring + par * BUF + cls * CS + i16) +
+                          (g >> 1);
+#pragma unroll
+      for (int qq = 0; qq < QS; qq++) {
+        const uint32_t* bq = b + qq * 8 * CS * 4;
+        const float a0 = val(bq[0]), a1 = val(bq[2]);
+#pragma unroll
+        for (int i = 0; i < TN; i++) {
+          const uint32_t* x = bq + (RT + 16 * i) * 4;
+          acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(a0, val(x[0]), acc[i], 0, 0, 0);
+          if constexpr (CH == 8)
+            acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(a1, val(x[2]), acc[i], 0, 0, 0);
+        }
+      }
+      lds_barrier();
+      par ^= 1;
+    }
+    // stage sg's group is summed: the tree's counter
+#pragma unroll
+    for (int i = 0; i < TN; i++) {
+      if (sg & 1) {
+        acc[i] = p0[i] + acc[i];
+        if (sg & 2) {
+          acc[i] = p1[i] + acc[i];
+          if (sg & 4) acc[i] = p2[i] + acc[i];
+          else p2[i] = acc[i];
+        } else {
+          p1[i] = acc[i];
+        }
+      } else {
+        p0[i] = acc[i];
+      }
+    }
+  }
+  // the classes' tiles through LDS (every wave has read the ring)
+  float* red = reinterpret_cast<float*>(sm);
+#pragma unroll
+  for (int i = 0; i < TN; i++)
+    *reinterpret_cast<v4f*>(red + (cls * TT + 16 * i + i16) * RS + 4 * g) = acc[i];
+  lds_barrier();
+  auto sum4 = [&](int tok, int r) {
+    const v4f* c = reinterpret_cast<const v4f*>(red + tok * RS + r);
+    constexpr int S = TT * RS / 4;
+    return ((c[0] + c[4 * S]) + (c[2 * S] + c[6 * S])) + ((c[S] + c[5 * S]) + (c[3 * S] + c[7 * S]));
+  };
+  if constexpr (MODE == 2) {
+    const int b = t / (RU / 4), r = 4 * (t % (RU / 4)), u = r0 + r;
+    if (b < TT && b < n && u < nrows) {
+      const v4f gt = sum4(b, r), up = sum4(b, RU + r);
+      uint16_t* o = static_cast<uint16_t*>(out) + (int64_t)b * ldo;
+#pragma unroll
+      for (int k = 0; k < 4; k++)
+        if (u + k < nrows)
+          o[il(u + k, og)] = bf16_bits(bf16r(silu_bf16(bf16r(gt[k])) * bf16r(up[k])));
+    }
+  } else {
+    const int b = t / (RT / 4), r = 4 * (t % (RT / 4));
+    if (b < TT && b < n) {
+      const v4f v = sum4(b, r);
+      float* o = static_cast<float*>(out) + (int64_t)b * ldo + r0 + r;
+#pragma unroll
+      for (int k = 0; k < 4; k++)
+        if (r0 + r + k < nrows) {
+          if constexpr (MODE == 0) o[k] = bf16r(v[k]);
+          else o[k] = bf16r(o[k] + bf16r(v[k]));
+        }
     }
   }
 }
@@ -1998,22 +2162,28 @@ extern "C" int lxm_dn_run(const lxm_dn_params* ph, const lxm_dn_params* pd, int 
   return (int)hipErrorInvalidValue;
 }
 
-// the batched prefill's row kernels (MODE 2: nrows units of W and W2): 64 tokens a workgroup share
-// its rows' unpacking (two products an operand); up to 32 tokens take one 32-token tile, with half
-// the registers and four workgroups a CU to stream the weights
+// the batched prefill's row kernels (MODE 2: nrows units of W and W2). Where the line
+// lies, measured over a layer's four products at 64 tokens, pb_ms took 94, 123, 66
+// and 33 us for the projections, SwiGLU, down_proj and out_proj, pb_mm 55, 87, and for the hidden rows (80
+// workgroups) as long as at 100 tokens, 104 and 50: the wide rows go to pb_mm from 33 tokens, the
+// hidden ones from 65.
 template <int G, int MODE, int TN>
-static void launch_mm(const uint16_t* W, const uint16_t* W2, int nrows, const uint16_t* X, int n,
+static void launch_ms(const uint16_t* W, const uint16_t* W2, int nrows, const uint16_t* X, int n,
                       void* out, int ldo, int og, hipStream_t st) {
-  constexpr int RU = MODE == 2 ? 16 : 32;
-  const int nrt = (nrows + RU - 1) / RU, ntt = (n + 32 * TN - 1) / (32 * TN);
-  hipLaunchKernelGGL((pb_mm<G, MODE, TN>), dim3((nrt + 7) / 8 * 8 * ntt), dim3(PBT), 0, st, W, W2,
-                     nrows, X, n, out, ldo, og, ntt);
+  constexpr int RU = MODE == 2 ? 8 : 16;
+  hipLaunchKernelGGL((pb_ms<G, MODE, TN>), dim3((nrows + RU - 1) / RU), dim3(NT), 0, st, W, W2,
+                     nrows, X, n, out, ldo, og);
 }
 template <int G, int MODE>
 static void launch_pb(const uint16_t* W, const uint16_t* W2, int nrows, const uint16_t* X, int n,
                       void* out, int ldo, int og, hipStream_t st) {
-  if (n <= 32) launch_mm<G, MODE, 1>(W, W2, nrows, X, n, out, ldo, og, st);
-  else launch_mm<G, MODE, 2>(W, W2, nrows, X, n, out, ldo, og, st);
+  if (n <= 16) return launch_ms<G, MODE, 1>(W, W2, nrows, X, n, out, ldo, og, st);
+  if (n <= 32) return launch_ms<G, MODE, 2>(W, W2, nrows, X, n, out, ldo, og, st);
+  if (n <= 64 && MODE == 1) return launch_ms<G, MODE, 4>(W, W2, nrows, X, n, out, ldo, og, st);
+  constexpr int RU = MODE == 2 ? 16 : 32;
+  const int nrt = (nrows + RU - 1) / RU, ntt = (n + 63) / 64;
+  hipLaunchKernelGGL((pb_mm<G, MODE>), dim3((nrt + 7) / 8 * 8 * ntt), dim3(PBT), 0, st, W, W2,
+                     nrows, X, n, out, ldo, og, ntt);
 }
 // (G of the hidden rows, live value dims, inter) = (40, 64, 144) or (4, 8, 8). A batch's delta rule
 // runs token by token (pb_gdn), or chunk by chunk (chunked: lxm_gdn_chunks, the

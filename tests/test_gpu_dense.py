@@ -145,10 +145,10 @@ def test_dense_prefill_small(cuda, T, seed):
     check_prefill(T, 6, seed=seed)
 
 
-@pytest.mark.parametrize("n", [1, 32, 33, 64, 65, 97])
+@pytest.mark.parametrize("n", [1, 16, 17, 32, 33, 64, 65, 97])
 def test_dense_prefill_token_tiles(cuda, n):
-    """Prompts at the row kernels' token tiles (32 tokens in one tile, 64 a workgroup beyond): a
-    whole tile, one past it, one token alone, a last workgroup of one tile and a token."""
+    """Prompts at the row kernels' token tiles (16, 32 or 64 tokens on 16-row tiles, 64 a workgroup
+    on 32-row tiles beyond): whole tiles, one past them, one token alone."""
     check_prefill(n + 1, 2, seed=3)
 
 
