@@ -477,6 +477,18 @@ __global__ __launch_bounds__(NT, 8) void pf_tile(const lxm_pf_params* __restrict
     for (int c = t; c < H; c += NT) st_col<BF>(p.h, b, H, c, V::get(HV, c));
 }
 
+// A candidate's key slots to evaluate (0: not a candidate), from the masks of its position and the
+// three before it
+__device__ __forceinline__ uint32_t cand_mask(int tp, uint32_t m0, uint32_t m1, uint32_t m2,
+                                              uint32_t m3, int reach, uint32_t allk) {
+  uint32_t kb = m0 & 0xffffu;
+  if (reach >= 1) kb |= m1 & 0xffffu;
+  if (reach >= 2) kb |= m2 & 0xffffu;
+  if (reach >= 3) kb |= m3 & 0xffffu;
+  if (tp < reach) kb |= allk;
+  return kb | (m0 & 0x80000000u);
+}
+
 // ---------------------------------------------------------------------------------------------
 // The candidates of layer L, in position order: positions whose query/key channels of some live
 // key head can be nonzero (a nonzero projection within the earliest tap's reach, or a window
@@ -525,13 +537,7 @@ __global__ __launch_bounds__(C_NT) void pf_compact(const lxm_pf_params* __restri
 #pragma unroll
     for (int i = 0; i < C_PER; i++) {
       const int tp = t0 + i;
-      uint32_t kb = m[i + 3] & 0xffffu;
-      if (reach >= 1) kb |= m[i + 2] & 0xffffu;
-      if (reach >= 2) kb |= m[i + 1] & 0xffffu;
-      if (reach >= 3) kb |= m[i] & 0xffffu;
-      if (tp < reach) kb |= allk;
-      kb |= m[i + 3] & 0x80000000u;
-      cm[i] = tp < T ? kb : 0u;
+      cm[i] = tp < T ? cand_mask(tp, m[i + 3], m[i + 2], m[i + 1], m[i], reach, allk) : 0u;
       n += cm[i] != 0u;
     }
     // exclusive scan of n over the workgroup
@@ -596,14 +602,29 @@ __device__ __forceinline__ float conv_y(const v4f P, const float* taps, int tok,
   return silu_rd<BF>(rd<BF>(y));
 }
 
-// One workgroup per candidate (grid-stride): the input norm's output at positions tok..tok-3
+// Workgroups per candidate, from the layer's candidates: one where they fill the 256 CUs, up to `most`
+// where they leave them idle (four each measured slower from 230 candidates on: 53 against 38 us for
+// pf_act, 22.3 against 18.8 for pf_out).
+__device__ __forceinline__ int parts_of(int count, int most) {
+  const int n = 256 / (count > 0 ? count : 1);
+  return n < 1 ? 1 : n < most ? n : most;
+}
+
+// parts_of() workgroups per candidate (grid-stride): the input norm's output at positions tok..tok-3
 // (lanes 0..3 of a tile-shaped vector in LDS), the query/key conv outputs of its key slots,
 // which slots are live, their l2norms; for the live slots' value heads the value channels' conv
-// outputs, the in_proj_z rows and beta; every slot's decay factor exp(g). LDS: the normed input
-// (64 KB), q/k per key slot (32 KB), the live word.
+// outputs, the in_proj_z rows and beta; every slot's decay factor exp(g). The parts share out the
+// value channels, each repeating the norm and the keys; part 0 writes the keys, the last part the
+// decays and betas. LDS: the normed input (64 KB), q/k per key slot (32 KB), the live word, the list.
+// OWN (T <= NT): every workgroup forms the candidate list itself, a position a thread, so that a
+// short call has no compaction launch (7.0 us, a workgroup's latency) before this one.
+// A call of few candidates is bound by one candidate's latency: with one workgroup for all its value
+// channels (8-16 rounds of dependent loads) 31.5 us a layer at 61 positions of the 37-layer
+// stack and 38.2 at 65,536 (230 candidates a layer), ACT_SMALL and ACT_LARGE with 8 and 4 parts.
 #define A_QK (16 * MAXH)
 #define A_MISC (A_QK + 4 * LXM_PF_MAXKS * 2 * KD)
-template <bool BF>
+#define A_LIST (A_MISC + 16)
+template <bool BF, bool OWN>
 __global__ __launch_bounds__(NT) void pf_act(const lxm_pf_params* __restrict__ pp, int L) {
   extern __shared__ __align__(16) uint8_t sm[];
   const lxm_pf_params& p = *pp;
@@ -616,29 +637,73 @@ __global__ __launch_bounds__(NT) void pf_act(const lxm_pf_params* __restrict__ p
   const float* w1 = tab<float>(p.blob, ly.w1_in);
   const void* cs = p.conv[L];
   const RecOff ro(ly.n_ks, ly.n_vs);
-  const int count = p.count[L];
-  for (int j = blockIdx.x; j < count; j += gridDim.x) {
-    const int tok = p.cand[j];
-    const uint32_t cm = p.cmask[j];
+  int count;
+  if constexpr (OWN) {
+    int32_t* lt = reinterpret_cast<int32_t*>(sm + A_LIST);
+    uint32_t* lm = reinterpret_cast<uint32_t*>(lt + NT);
+    int32_t* wn = lt + 2 * NT;
+    const int T = p.T, reach = ly.reach;
+    const uint32_t allk = ly.n_ks >= 32 ? 0xffffffffu : ((1u << ly.n_ks) - 1u);
+    uint32_t m[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const uint32_t v = p.mask[t - i < 0 ? 0 : t - i < T ? t - i : T - 1];
+      m[i] = t - i >= 0 && t < T ? v : 0u;
+    }
+    const uint32_t cm = t < T ? cand_mask(t, m[0], m[1], m[2], m[3], reach, allk) : 0u;
+    const unsigned long long bal = __ballot(cm != 0u);
+    if (lane == 0) wn[wv] = __popcll(bal);
+    __syncthreads();
+    int base = 0;
+    count = 0;
+#pragma unroll
+    for (int w = 0; w < NW; w++) {
+      base += w < wv ? wn[w] : 0;
+      count += wn[w];
+    }
+    if (cm != 0u) {
+      const int o = base + __popcll(bal & ((1ull << lane) - 1ull));
+      lt[o] = t;
+      lm[o] = cm;
+    }
+    if (blockIdx.x == 0 && t == 0) p.count[L] = count;
+    __syncthreads();
+  } else {
+    count = p.count[L];
+  }
+  const int parts = parts_of(count, 8);
+  for (int item = blockIdx.x; item < count * parts; item += gridDim.x) {
+    const int j = item / parts, part = item % parts;
+    const int tok = OWN ? reinterpret_cast<const int32_t*>(sm + A_LIST)[j] : p.cand[j];
+    const uint32_t cm = OWN ? reinterpret_cast<const uint32_t*>(sm + A_LIST)[NT + j] : p.cmask[j];
     uint8_t* rec = p.recs + (int64_t)j * ly.rec_bytes;
     float rr[4];
 #pragma unroll
     for (int s = 0; s < 4; s++) rr[s] = tok - s >= 0 ? p.r1[tok - s] : 0.0f;
     // positions tok - s, s = 0..3: lane l0 - s of tile tok / 4 for s <= l0, else lane l0 - s + 4 of
-    // the tile before (tok / 4 and l0 the same for the whole workgroup), read as columns
+    // the tile before (tok / 4 and l0 the same for the whole workgroup), read as columns, all
+    // requested before any is used (a column past H: the last one's, unused)
     const int64_t b0 = tok >> 2;
     const int l0 = tok & 3;
-    for (int c = t; c < H; c += NT) {
-      const v4f c0 = ld_col<BF>(p.h, b0, H, c);
-      const v4f c1 = l0 < 3 && b0 > 0 ? ld_col<BF>(p.h, b0 - 1, H, c) : v4f{0.0f, 0.0f, 0.0f, 0.0f};
-      const float w = w1[c];
+    const bool two = l0 < 3 && b0 > 0;
+    v4f c0[MAXH / NT], c1[MAXH / NT];
+    float w[MAXH / NT];
+#pragma unroll
+    for (int k = 0; k < MAXH / NT; k++) {
+      const int c = t + k * NT < H ? t + k * NT : H - 1;
+      c0[k] = ld_col<BF>(p.h, b0, H, c);
+      c1[k] = ld_col<BF>(p.h, two ? b0 - 1 : b0, H, c);
+      w[k] = w1[c];
+    }
+#pragma unroll
+    for (int k = 0; k < MAXH / NT; k++) {
       v4f x;
 #pragma unroll
       for (int s = 0; s < 4; s++) {
-        const float h = s <= l0 ? c0[l0 - s] : c1[l0 - s + 4];
-        x[s] = tok - s >= 0 ? rd<BF>((h * rr[s]) * w) : 0.0f;
+        const float h = s <= l0 ? c0[k][l0 - s] : c1[k][l0 - s + 4];
+        x[s] = tok - s >= 0 ? rd<BF>((h * rr[s]) * w[k]) : 0.0f;
       }
-      XN[c] = x;
+      if (t + k * NT < H) XN[t + k * NT] = x;
     }
     for (int i = t; i < ly.n_ks * 2 * KD; i += NT) QK[i] = 0.0f;
     if (t == 0) *live_s = 0u;
@@ -674,7 +739,7 @@ __global__ __launch_bounds__(NT) void pf_act(const lxm_pf_params* __restrict__ p
       for (int i = 0; i < 4; i++) {
         float v = rd<BF>(xs[i] * inv);
         if (!isk) v = v * 0.0625f;
-        o[lane + 64 * i] = v;
+        if (part == 0) o[lane + 64 * i] = v;
       }
     }
     __syncthreads();
@@ -684,7 +749,7 @@ __global__ __launch_bounds__(NT) void pf_act(const lxm_pf_params* __restrict__ p
     const lxm_row* zr = tab<lxm_row>(p.blob, ly.zrow);
     float* rv = reinterpret_cast<float*>(rec + ro.v);
     float* rz = reinterpret_cast<float*>(rec + ro.z);
-    for (int i = t; i < ly.n_vs * VD; i += NT) {
+    for (int i = part * NT + t; i < ly.n_vs * VD; i += parts * NT) {
       const lxm_pf_vs sv = vs[i >> 7];
       if (sv.kslot < 0 || !((live >> sv.kslot) & 1u)) continue;
       const lxm_pf_vc c = vc[i];
@@ -696,7 +761,7 @@ __global__ __launch_bounds__(NT) void pf_act(const lxm_pf_params* __restrict__ p
     }
     const lxm_row* br = tab<lxm_row>(p.blob, ly.brow);
     const lxm_pf_dec* dc = tab<lxm_pf_dec>(p.blob, ly.dec);
-    for (int i = t; i < ly.n_vs; i += NT) {
+    for (int i = t; i < ly.n_vs && part == parts - 1; i += NT) {
       const lxm_pf_vs sv = vs[i];
       float e = 1.0f;
       if (sv.dslot >= 0) {
@@ -712,7 +777,7 @@ __global__ __launch_bounds__(NT) void pf_act(const lxm_pf_params* __restrict__ p
         reinterpret_cast<float*>(rec + ro.b)[i] = rd<BF>(sigmoid(rd<BF>(dot1<BF>(ent + bb.start, bb.len, sm))));
       }
     }
-    if (t == 0) {
+    if (t == 0 && part == 0) {
       reinterpret_cast<int32_t*>(rec)[0] = tok;
       reinterpret_cast<uint32_t*>(rec)[1] = live;
     }
@@ -722,40 +787,53 @@ __global__ __launch_bounds__(NT) void pf_act(const lxm_pf_params* __restrict__ p
 
 // ---------------------------------------------------------------------------------------------
 // The conv windows the call leaves (causal_conv1d_update's state after the last position: each
-// channel's last 4 projections, TF:199-216), for every channel of layer L. Runs while p->h holds
-// the layer's input and after pf_act has read the windows the call started from.
+// channel's last 4 projections, TF:199-216), for channel c of layer L. Runs while p->h holds the
+// layer's input and after pf_act has read the windows the call started from: in pf_delta's launch,
+// whose few long waves leave the CUs to it (as a launch of its own 6.7-8.4 us a layer).
 template <bool BF>
-__global__ __launch_bounds__(256) void pf_tail(const lxm_pf_params* __restrict__ pp, int L) {
-  const lxm_pf_params& p = *pp;
-  const lxm_pf_layer& ly = p.layers[L];
-  const int c = blockIdx.x * 256 + threadIdx.x, H = p.hidden, T = p.T;
+__device__ __forceinline__ void tail_chan(const lxm_pf_params& p, const lxm_pf_layer& ly, int L,
+                                          int c) {
+  const int H = p.hidden, T = p.T;
   if (c >= p.n_conv) return;
   const lxm_pf_ent* ent = tab<lxm_pf_ent>(p.blob, ly.ent);
   const float* w1 = tab<float>(p.blob, ly.w1_in);
-  const lxm_row row = tab<lxm_row>(p.blob, ly.cc)[c];
+  const lxm_row row = gld(tab<lxm_row>(p.blob, ly.cc) + c);
   void* cs = p.conv[L];
-  // one pass over the channel's entries forms the four window sums (each in entry order); the
-  // positions T-4..T-1 are lanes of the last tile and the one before it, read as columns
+  // one pass over the channel's entries, four at a time (four padding entries follow the table),
+  // forms the four window sums (each in entry order); the positions T-4..T-1 are lanes of the
+  // last tile and the one before it, read as columns
   const int64_t b0 = (T - 1) >> 2;
   const int l0 = (T - 1) & 3;
+  const bool two = l0 < 3 && b0 > 0;
   float r[4], s[4];
 #pragma unroll
   for (int j = 0; j < 4; j++) {
     r[j] = T - 4 + j >= 0 ? p.r1[T - 4 + j] : 0.0f;
     s[j] = 0.0f;
   }
-  for (int k = 0; k < row.len; k++) {
-    const lxm_pf_ent e = ent[row.start + k];
-    const int col = e.off >> 4;
-    const float w = w1[col];
-    const v4f c0 = ld_col<BF>(p.h, b0, H, col);
-    const v4f c1 = l0 < 3 && b0 > 0 ? ld_col<BF>(p.h, b0 - 1, H, col) : v4f{0.0f, 0.0f, 0.0f, 0.0f};
+  for (int k0 = 0; k0 < row.len; k0 += 4) {
+    lxm_pf_ent e[4];
+    v4f c0[4], c1[4];
+    float w[4];
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-      const int d = 3 - j;  // position T-1-d
-      const float h = d <= l0 ? c0[l0 - d] : c1[l0 - d + 4];
-      if (T - 4 + j >= 0) s[j] = acc<BF>(s[j], rd<BF>((h * r[j]) * w), e.w);
+    for (int k = 0; k < 4; k++) e[k] = gld(ent + row.start + (k0 + k < row.len ? k0 + k : k0));
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      const int col = e[k].off >> 4;
+      w[k] = w1[col];
+      c0[k] = ld_col<BF>(p.h, b0, H, col);
+      c1[k] = ld_col<BF>(p.h, two ? b0 - 1 : b0, H, col);
     }
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+      if (k0 + k < row.len) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+          const int d = 3 - j;  // position T-1-d
+          const float h = d <= l0 ? c0[k][l0 - d] : c1[k][l0 - d + 4];
+          if (T - 4 + j >= 0) s[j] = acc<BF>(s[j], rd<BF>((h * r[j]) * w[k]), e[k].w);
+        }
+      }
   }
   float win[4];
 #pragma unroll
@@ -811,7 +889,8 @@ __device__ __forceinline__ DeltaIn delta_in(const uint8_t* rec, const RecOff& ro
   return d;
 }
 // the 16 block sums of this lane's column, from +0 in block order (every lane of the column
-// gets the same sum)
+// gets the same sum). (Across the lanes by 15 DPP adds, each with its wait states, measured slower:
+// 242 against 216 us a layer at 230 candidates.)
 __device__ __forceinline__ float col_sum16(float* red, int c, int b, float x) {
   red[16 * c + b] = x;
   __atomic_signal_fence(__ATOMIC_SEQ_CST);
@@ -889,11 +968,15 @@ __device__ __forceinline__ void delta_step(const DeltaIn& cur, float (&s)[16], f
 }
 
 template <bool BF>
-__global__ __launch_bounds__(64) void pf_delta(const lxm_pf_params* __restrict__ pp, int L) {
+__global__ __launch_bounds__(64) void pf_delta(const lxm_pf_params* __restrict__ pp, int L, int nd) {
   __shared__ __align__(16) float red[DCW * 16];
   __shared__ __align__(16) float kqs[2 * KQ_Q];  // a live step's k and q (rows of 20)
   const lxm_pf_params& p = *pp;
   const lxm_pf_layer& ly = p.layers[L];
+  if ((int)blockIdx.x >= nd) {  // the windows' workgroups, 64 channels each
+    tail_chan<BF>(p, ly, L, ((int)blockIdx.x - nd) * 64 + threadIdx.x);
+    return;
+  }
   const int lane = threadIdx.x, c = lane >> 4, b = lane & 15;
   // a slot's DWS workgroups on one XCD (workgroups are dealt to the 8 XCDs in turn): the slot's
   // records are then fetched into one L2, and its columns' outputs merge in it
@@ -950,6 +1033,9 @@ __global__ __launch_bounds__(64) void pf_delta(const lxm_pf_params* __restrict__
 // (TF:541-543, :777-779): per residual row the terms over every value dim in ascending order,
 // rounded once (lx/lx/fast.py:349-361), then h = D(h + that). Heads that did not run add nothing
 // (their output is exactly 0 and the oracle skips zero inputs). One workgroup per candidate.
+// parts_of() workgroups share a candidate's residual rows, each forming the norms; a wave's heads come
+// four at a time, their inputs requested together (one workgroup a candidate, a head at a time: 15.2 us
+// a layer at 61 positions, 8.6 now).
 template <bool BF>
 __global__ __launch_bounds__(NT) void pf_out(const lxm_pf_params* __restrict__ pp, int L) {
   extern __shared__ __align__(16) uint8_t sm[];
@@ -963,8 +1049,9 @@ __global__ __launch_bounds__(NT) void pf_out(const lxm_pf_params* __restrict__ p
   const lxm_pf_ent* ent = tab<lxm_pf_ent>(p.blob, ly.ent);
   const float* gwp = tab<float>(p.blob, ly.gnorm);
   const float gw0 = gwp[lane], gw1 = gwp[lane + 64], geps = ly.geps;
-  const int count = p.count[L], n_vs = ly.n_vs;
-  for (int j = blockIdx.x; j < count; j += gridDim.x) {
+  const int count = p.count[L], n_vs = ly.n_vs, parts = parts_of(count, 4);
+  for (int item = blockIdx.x; item < count * parts; item += gridDim.x) {
+    const int j = item / parts, part = item % parts;
     const uint8_t* rec = p.recs + (int64_t)j * ly.rec_bytes;
     const int tok = reinterpret_cast<const int32_t*>(rec)[0];
     const int32_t* pr = reinterpret_cast<const int32_t*>(rec + ro.pr);
@@ -972,29 +1059,44 @@ __global__ __launch_bounds__(NT) void pf_out(const lxm_pf_params* __restrict__ p
     const float* z = reinterpret_cast<const float*>(rec + ro.z);
     if (t == 0) any_s = 0;
     __syncthreads();
-    for (int v = wv; v < n_vs; v += NT / 64) {
-      float y0 = 0.0f, y1 = 0.0f;
-      if (pr[v] == 2) {
-        const float o0 = o[v * VD + lane], o1 = o[v * VD + lane + 64];
-        const float z0 = z[v * VD + lane], z1 = z[v * VD + lane + 64];
-        float ss = 0.0f;
-        ss = ss + o0 * o0;
-        ss = ss + o1 * o1;
-        ss = sum64(ss);
-        const float rr = rsqrt_(ss / (float)VD + geps);
-        y0 = rd<BF>(rd<BF>(gw0 * rd<BF>(o0 * rr)) * silu(z0));
-        y1 = rd<BF>(rd<BF>(gw1 * rd<BF>(o1 * rr)) * silu(z1));
-        if (lane == 0) any_s = 1;
+    for (int v0 = wv; v0 < n_vs; v0 += 4 * (NT / 64)) {
+      int ran[4];
+      float o0[4], o1[4], z0[4], z1[4];
+#pragma unroll
+      for (int u = 0; u < 4; u++) {  // (a head that did not run: values of the record, unused)
+        const int v = v0 + u * (NT / 64) < n_vs ? v0 + u * (NT / 64) : v0;
+        ran[u] = pr[v];
+        o0[u] = o[v * VD + lane];
+        o1[u] = o[v * VD + lane + 64];
+        z0[u] = z[v * VD + lane];
+        z1[u] = z[v * VD + lane + 64];
       }
-      ON[v * VD + lane] = y0;
-      ON[v * VD + lane + 64] = y1;
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        const int v = v0 + u * (NT / 64);
+        if (v >= n_vs) break;
+        float y0 = 0.0f, y1 = 0.0f;
+        if (ran[u] == 2) {
+          float ss = 0.0f;
+          ss = ss + o0[u] * o0[u];
+          ss = ss + o1[u] * o1[u];
+          ss = sum64(ss);
+          const float rr = rsqrt_(ss / (float)VD + geps);
+          y0 = rd<BF>(rd<BF>(gw0 * rd<BF>(o0[u] * rr)) * silu(z0[u]));
+          y1 = rd<BF>(rd<BF>(gw1 * rd<BF>(o1[u] * rr)) * silu(z1[u]));
+          if (lane == 0) any_s = 1;
+        }
+        ON[v * VD + lane] = y0;
+        ON[v * VD + lane + 64] = y1;
+      }
     }
     __syncthreads();
     if (any_s) {
-      for (int i = t; i < ly.n_orows; i += NT) {
-        const lxm_pf_drow r = orows[i];
+      for (int i = part * NT + t; i < ly.n_orows; i += parts * NT) {
+        const lxm_pf_drow r = gld(orows + i);
+        const float h = ld_el<BF>(p.h, H, tok, r.row);
         const float y = rd<BF>(dot1<BF>(ent + r.start, r.len, sm));
-        st_el<BF>(p.h, H, tok, r.row, rd<BF>(ld_el<BF>(p.h, H, tok, r.row) + y));
+        st_el<BF>(p.h, H, tok, r.row, rd<BF>(h + y));
       }
     }
     __syncthreads();
@@ -1157,7 +1259,7 @@ template <bool BF>
 static int tile_lds(int H, int n_units_max) {
   return x_xm<BF>(H) + TV<BF>::B * (n_units_max + 1);
 }
-#define ACT_LDS (A_MISC + 16)
+#define ACT_LDS (A_LIST + 8 * NT + 4 * NW)
 #define ACT_GRID 1024
 #define OUT_GRID 1024
 
@@ -1174,20 +1276,30 @@ static hipError_t run_layers(const lxm_pf_params* ph, const lxm_pf_params* pd, i
   for (int L = l0; L < l1; L++) umax = ph->layers_host[L].n_units > umax ? ph->layers_host[L].n_units : umax;
   const int xl = tile_lds<BF>(ph->hidden, umax);
   hipError_t e = lds_attr((const void*)pf_tile<BF>, xl);
-  if (e == hipSuccess) e = lds_attr((const void*)pf_act<BF>, ACT_LDS);
+  if (e == hipSuccess) e = lds_attr((const void*)pf_act<BF, true>, ACT_LDS);
+  if (e == hipSuccess) e = lds_attr((const void*)pf_act<BF, false>, ACT_LDS);
   if (e == hipSuccess) e = lds_attr((const void*)pf_out<BF>, 4 * VD * LXM_PF_MAXVS + 16);
   if (e != hipSuccess) return e;
+  // pf_act lists the candidates itself where a position a thread suffices; a short call cannot have
+  // more workgroups' work than its positions'
+  const int T = ph->T;
+  const bool own = T <= NT;
+  const int ag = T < ACT_GRID / 8 ? T * 8 : ACT_GRID, og = T < OUT_GRID / 4 ? T * 4 : OUT_GRID;
   for (int L = l0; L < l1; L++) {
     const lxm_pf_layer& ly = ph->layers_host[L];
     hipLaunchKernelGGL(pf_tile<BF>, dim3(ntiles), dim3(NT), xl, st, pd, L == l0 ? -1 : L - 1, L);
-    hipLaunchKernelGGL(pf_compact, dim3(1), dim3(C_NT), 0, st, pd, L);
-    hipLaunchKernelGGL(pf_act<BF>, dim3(ACT_GRID), dim3(NT), ACT_LDS, st, pd, L);
-    hipLaunchKernelGGL(pf_tail<BF>, dim3((ph->n_conv + 255) / 256), dim3(256), 0, st, pd, L);
-    // (DWS one-wave workgroups per value-head slot, DCW state columns each, a slot's on one XCD)
+    if (own) {
+      hipLaunchKernelGGL((pf_act<BF, true>), dim3(ag), dim3(NT), ACT_LDS, st, pd, L);
+    } else {
+      hipLaunchKernelGGL(pf_compact, dim3(1), dim3(C_NT), 0, st, pd, L);
+      hipLaunchKernelGGL((pf_act<BF, false>), dim3(ag), dim3(NT), ACT_LDS, st, pd, L);
+    }
+    // (DWS one-wave workgroups per value-head slot, DCW state columns each, a slot's on one XCD;
+    // after them the conv windows')
+    const int nd = 8 * DWS * ((ly.n_vs + 7) / 8);
+    hipLaunchKernelGGL(pf_delta<BF>, dim3(nd + (ph->n_conv + 63) / 64), dim3(64), 0, st, pd, L, nd);
     if (ly.n_vs > 0)
-      hipLaunchKernelGGL(pf_delta<BF>, dim3(8 * DWS * ((ly.n_vs + 7) / 8)), dim3(64), 0, st, pd, L);
-    if (ly.n_vs > 0)
-      hipLaunchKernelGGL(pf_out<BF>, dim3(OUT_GRID), dim3(NT), 4 * VD * ly.n_vs + 16, st, pd, L);
+      hipLaunchKernelGGL(pf_out<BF>, dim3(og), dim3(NT), 4 * VD * ly.n_vs + 16, st, pd, L);
   }
   hipLaunchKernelGGL(pf_tile<BF>, dim3(ntiles), dim3(NT), xl, st, pd, l1 - 1, -1);
   return hipGetLastError();

@@ -89,6 +89,14 @@ def test_prefill_small(cuda):
     check("small", _toks("small", 37))
 
 
+@pytest.mark.parametrize("name,T", [("small", 511), ("small", 512), ("small", 513), ("small_fp32", 512),
+                                    ("c1", 700)])
+def test_prefill_candidate_lists(cuda, name, T):
+    """Around the 512 positions up to which the candidate inputs' kernel lists the candidates itself;
+    layers of many candidates (one workgroup each) and of few (up to eight, up to four)."""
+    check(name, _toks(name, T), per_layer=False)
+
+
 def test_prefill_small_fp32(cuda):
     check("small_fp32", _toks("small_fp32", 30))
 
