@@ -740,7 +740,7 @@ def dense_cpu_stock(dm, toks, n_prompt: int, max_steps: int, budget_s: float) ->
 
 def dense_leg(args, dev) -> dict:
     """Benchmark config 4: the dense padded text-view stack; a prompt of n_prefill seeded uniform
-    tokens from a zero state (batched: lxm_dn_prefill over all but the last, then one step;
+    tokens from a zero state (batched: lxm_dn_prefill_n over all but the last, then one step;
     else n_prefill forced steps), then n_steps greedy steps, timed (HIP events on the stream)."""
     import numpy as np
     import torch
@@ -761,7 +761,7 @@ def dense_leg(args, dev) -> dict:
     toks = np.random.default_rng(spec.seed).integers(0, spec.vocab, n_prefill).tolist()
     t = time.perf_counter()
     if args.dn_batched:
-        dd.prefill(toks[:-1])  # lxm_dn_prefill: the same states as forced steps, bit for bit
+        dd.prefill(toks[:-1])  # lxm_dn_prefill_n: the same states as forced steps, bit for bit
         p1 = dd.run(toks[-1:], 1, graph=graph)
     else:
         p1 = dd.run(toks, n_prefill, graph=graph)
@@ -799,7 +799,7 @@ def dense_leg(args, dev) -> dict:
         ch_s = time.perf_counter() - t
         chunked = {"tokens": n_prefill, "s": round(ch_s, 3), "tok_s": round(n_prefill / ch_s, 1),
                    "first_prediction_equal": bool(pc[0] == p1[-1]),
-                   "mode": "lxm_dn_prefill_chunked (chunks of 64, lxm_gdn_chunk on MFMA) + one step"}
+                   "mode": "lxm_dn_prefill_n, chunked (chunks of 64, lxm_gdn_chunks on MFMA) + one step"}
         log(f"[bench] c4: chunked prompt of {n_prefill} tokens in {ch_s:.2f}s")
         del dd2, c2
     H, I, nk, kl, rl = spec.hidden, spec.inter, spec.nk, spec.kd_live, spec.r_live
@@ -818,6 +818,7 @@ def dense_leg(args, dev) -> dict:
     # fused multiply-adds per prompt token: every live weight of every layer once
     fma_tok = d.n_layers * ((2 * nk * kl + 2 * nvr + 2 * nk * rl) * H + H * nvr + 3 * I * H)
     pf_rate = 2 * fma_tok * n_prefill / pre_s / 1e12
+    pf_peak = FP32_PEAK_TFLOPS if args.dn_batched else FP32_PEAK_TFLOPS / 2
     out = {"metric": "dense padded decode tok/s, 24-layer text-view stack, 1 MI355X",
            "value": round(tok_s, 1), "unit": "tok/s",
            "ms_per_token": round(1e3 / tok_s, 4),
@@ -827,15 +828,18 @@ def dense_leg(args, dev) -> dict:
                      "note": "lxm_dn_step captured once and replayed per token"},
            "prefill": {"tokens": n_prefill, "s": round(pre_s, 2),
                        "tok_s": round(n_prefill / pre_s, 1),
-                       "mode": "lxm_dn_prefill (batches of 16) + one step" if args.dn_batched
+                       "mode": "lxm_dn_prefill_n (batches of 2,048) + one step" if args.dn_batched
                                else "forced steps",
-                       # the prompt's row sums are fp32 fused ops on the VALU (bf16 x bf16
-                       # products, summed in the decode's order); packed fp32 is not used, so
-                       # the vector rate available is half the published fp32 peak
-                       "roofline": {"bound": "valu", "achieved": round(pf_rate, 2),
-                                    "peak": FP32_PEAK_TFLOPS / 2, "unit": "TFLOP/s",
-                                    "frac": round(pf_rate / (FP32_PEAK_TFLOPS / 2), 4),
-                                    "peak_note": "half of the published 157.3 TFLOP/s fp32 peak: "
+                       # the prompt's row sums are fp32 fused ops (bf16 x bf16 products, summed in the
+                       # decode's order), on the fp32 matrix cores in batches (forced steps: the
+                       # vector unit, without packed fp32: half the published peak)
+                       "roofline": {"bound": "mfma_f32" if args.dn_batched else "valu",
+                                    "achieved": round(pf_rate, 2),
+                                    "peak": pf_peak, "unit": "TFLOP/s",
+                                    "frac": round(pf_rate / pf_peak, 4),
+                                    "peak_note": "the published 157.3 TFLOP/s fp32 matrix peak"
+                                                 if args.dn_batched else
+                                                 "half of the published 157.3 TFLOP/s fp32 peak: "
                                                  "no packed fp32 ops",
                                     "flops_per_token": 2 * fma_tok}},
            "config": {"workload": "c4: 24 layers, hidden 2560, 16 key heads (256, 128 live), 128 "
@@ -903,9 +907,9 @@ def make_parser() -> argparse.ArgumentParser:
     ap.add_argument("--dn-graph", type=int, default=1,
                     help="1: the dense steps replayed from a captured graph; 0: launched eagerly")
     ap.add_argument("--dn-batched", type=int, default=1,
-                    help="config 4's prompt through lxm_dn_prefill (0: as forced steps)")
+                    help="config 4's prompt through lxm_dn_prefill_n (0: as forced steps)")
     ap.add_argument("--dn-chunked", type=int, default=1,
-                    help="1: also time the prompt through lxm_dn_prefill_chunked; 0: skip it")
+                    help="1: also time the prompt in the chunked form; 0: skip it")
     ap.add_argument("--dn-persistent", type=int, default=1,
                     help="1: also time the persistent run (lxm_dn_run); 0: skip it")
     return ap

@@ -622,7 +622,7 @@ __device__ __forceinline__ int parts_of(int count, int most) {
 // short call has no compaction launch (7.0 us, a workgroup's latency) before this one.
 // A call of few candidates is bound by one candidate's latency: with one workgroup for all its value
 // channels (8-16 rounds of dependent loads) 31.5 us a layer at 61 positions of the 37-layer
-// stack and 38.2 at 65,536 (230 candidates a layer), ACT_SMALL and ACT_LARGE with 8 and 4 parts.
+// stack, 12.0 with 8 parts.
 #define A_QK (16 * MAXH)
 #define A_MISC (A_QK + 4 * LXM_PF_MAXKS * 2 * KD)
 #define A_LIST (A_MISC + 16)
@@ -667,6 +667,10 @@ __global__ __launch_bounds__(NT) void pf_act(const lxm_pf_params* __restrict__ p
       const int o = base + __popcll(bal & ((1ull << lane) - 1ull));
       lt[o] = t;
       lm[o] = cm;
+      if (blockIdx.x == 0) {
+        p.cand[o] = t;
+        p.cmask[o] = cm;
+      }
     }
     if (blockIdx.x == 0 && t == 0) p.count[L] = count;
     __syncthreads();
