@@ -1685,7 +1685,10 @@ __global__ __launch_bounds__(NT) void pb_ms(const uint16_t* __restrict__ W,
       lds_barrier();
       par ^= 1;
     }
-    // stage sg's group is summed: the tree's counter
+    // stage sg's group is summed: the tree's counter. (The last MFMAs are waited for here: their
+    // results are first read inside branches, where the compiler has been seen to leave out the wait.)
+#pragma unroll
+    for (int i = 0; i < TN; i++) asm volatile("s_nop 15" : "+v"(acc[i]));
 #pragma unroll
     for (int i = 0; i < TN; i++) {
       if (sg & 1) {
@@ -2179,7 +2182,9 @@ static void launch_pb(const uint16_t* W, const uint16_t* W2, int nrows, const ui
                       void* out, int ldo, int og, hipStream_t st) {
   if (n <= 16) return launch_ms<G, MODE, 1>(W, W2, nrows, X, n, out, ldo, og, st);
   if (n <= 32) return launch_ms<G, MODE, 2>(W, W2, nrows, X, n, out, ldo, og, st);
-  if (n <= 64 && MODE == 1) return launch_ms<G, MODE, 4>(W, W2, nrows, X, n, out, ldo, og, st);
+  if constexpr (MODE == 1) {
+    if (n <= 64) return launch_ms<G, MODE, 4>(W, W2, nrows, X, n, out, ldo, og, st);
+  }
   constexpr int RU = MODE == 2 ? 16 : 32;
   const int nrt = (nrows + RU - 1) / RU, ntt = (n + 63) / 64;
   hipLaunchKernelGGL((pb_mm<G, MODE>), dim3((nrt + 7) / 8 * 8 * ntt), dim3(PBT), 0, st, W, W2,
