@@ -43,9 +43,9 @@ typedef struct lxm_chunk_io {
   int32_t o_bf16;  /* 1: o rounded to bf16 (the stock casts the output to the model dtype) */
 } lxm_chunk_io;
 
-/* One chunk of every slot on stream (one workgroup per slot and 16 state columns). q, k, v and S
-   are read 16 bytes at a time: each must be 16-byte aligned and qk_ts, qk_hs and v_ts multiples of
-   4. Returns a hipError_t (hipErrorInvalidValue for sizes outside the limits above or a misaligned
+/* One chunk of every slot on stream (one workgroup per slot and 16 state columns; past 32 slots, 32
+   columns). q, k, v and S are read 16 bytes at a time: each must be 16-byte aligned and qk_ts,
+   qk_hs and v_ts multiples of 4. Returns a hipError_t (hipErrorInvalidValue for sizes outside the limits above or a misaligned
    pointer or stride). */
 int lxm_gdn_chunk(const lxm_chunk_io* io, void* stream);
 

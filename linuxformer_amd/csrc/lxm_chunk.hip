@@ -355,7 +355,7 @@ __device__ __forceinline__ v4f chunk_step(StepLds& st, const float* k, int nkt, 
 __device__ __forceinline__ float* state_of(const lxm_chunk_io& io, int h, int c0) {
   return io.S + ((size_t)(h / io.rl) * io.rfull + h % io.rl) * 256 * VD + c0;
 }
-__device__ __forceinline__ void load_state(const float* S, int nkt, StepLds& st, v4f (&s)[2]) {
+__device__ __forceinline__ void load_state(const float* S, int nkt, v4f (&s)[2]) {
   const int w = wave(), lane = threadIdx.x & 63, i16 = lane & 15, g = lane >> 4;
 #pragma unroll
   for (int j = 0; j < 2; j++) {
@@ -364,8 +364,12 @@ __device__ __forceinline__ void load_state(const float* S, int nkt, StepLds& st,
 #pragma unroll
       for (int r = 0; r < 4; r++) s[j][r] = S[(size_t)(16 * (2 * w + j) + 4 * g + r) * VD + i16];
     }
-    st_b(st.s[2 * w + j], s[j]);
   }
+}
+__device__ __forceinline__ void stage_state(StepLds& st, const v4f (&s)[2]) {
+  const int w = wave();
+#pragma unroll
+  for (int j = 0; j < 2; j++) st_b(st.s[2 * w + j], s[j]);
 }
 __device__ __forceinline__ void store_state(float* S, int nkt, const v4f (&s)[2]) {
   const int w = wave(), lane = threadIdx.x & 63, i16 = lane & 15, g = lane >> 4;
@@ -386,12 +390,14 @@ __device__ __forceinline__ void store_o(const lxm_chunk_io& io, int h, int c0, i
       io.o[(p0 + i) * io.o_ts + (int64_t)h * VD + c0 + i16] = io.o_bf16 ? bf16r(o[r]) : o[r];
   }
 }
-// (workgroups are dealt to the 8 XCDs in turn: a head's 8 column groups on one of them, whose L2
-// then holds its keys, queries, T and A2)
+// (workgroups are dealt to the 8 XCDs in turn: a head's column groups, NB blocks of VT columns each, on
+// one of them, whose L2 then holds its keys, queries, T and A2)
+template <int NB>
 __device__ __forceinline__ bool head_cols(int n_slots, int& h, int& c0) {
+  constexpr int G = VD / (VT * NB);
   const int x = blockIdx.x & 7, j = blockIdx.x >> 3;
-  h = x + 8 * (j / (VD / VT));
-  c0 = (j % (VD / VT)) * VT;
+  h = x + 8 * (j / G);
+  c0 = (j % G) * VT * NB;
   return h < n_slots;
 }
 
@@ -445,7 +451,7 @@ __global__ __launch_bounds__(CT, 1) void chunk_run(lxm_chunk_io io, int T, int c
                                                    const float* ws) {
   __shared__ RunLds l;
   int h, c0;
-  if (!head_cols(io.n_slots, h, c0)) return;
+  if (!head_cols<1>(io.n_slots, h, c0)) return;
   const int w = wave(), lane = threadIdx.x & 63, i16 = lane & 15, g = lane >> 4;
   const int nkt = io.kl / 16, kh = h / io.rl, row = 16 * w + i16;
   float* S = state_of(io, h, c0);
@@ -476,7 +482,8 @@ __global__ __launch_bounds__(CT, 1) void chunk_run(lxm_chunk_io io, int T, int c
     }
     el = x[WS_V + 2 * C];
   };
-  load_state(S, nkt, l.st, s);
+  load_state(S, nkt, s);
+  stage_state(l.st, s);
   get_kq(0);
   get_rest(0);
   lds_barrier();
@@ -503,18 +510,19 @@ __global__ __launch_bounds__(CT, 1) void chunk_run(lxm_chunk_io io, int T, int c
   store_state(S, nkt, s);
 }
 
-// one chunk of every head: A2, T and W repeated by each of a head's 8 workgroups, each with its own
-// columns of U
+// one chunk of every head: A2, T and W repeated by each of a head's VD / (VT NB) workgroups, each with
+// its own columns of U and its NB steps one after the other (one block's tiles in LDS at a time)
+template <int NB>
 __global__ __launch_bounds__(CT, 1) void chunk_one(lxm_chunk_io io) {
   extern __shared__ __align__(16) uint8_t smem_raw[];
   OneLds& l = *reinterpret_cast<OneLds*>(smem_raw);
   int h, c0;
-  if (!head_cols(io.n_slots, h, c0)) return;
+  if (!head_cols<NB>(io.n_slots, h, c0)) return;
   const int w = wave(), lane = threadIdx.x & 63, i16 = lane & 15, g = lane >> 4;
   const int nkt = io.kl / 16, n = io.n, row = 16 * w + i16;
   const bool mine = 4 * (int)(threadIdx.x & 31) < io.kl;
   float* S = state_of(io, h, c0);
-  v4f kv[C / 8], s[2], vb[4], f[4];
+  v4f kv[C / 8], s[NB][2], vb[NB][4], f[4];
   if (mine) {
     load_rows(io.k, io.qk_ts, (int64_t)(h / io.rl) * io.qk_hs, n, kv);
   } else {  // (dims past kl: zero in every product)
@@ -525,13 +533,17 @@ __global__ __launch_bounds__(CT, 1) void chunk_one(lxm_chunk_io io) {
     });
   }
 #pragma unroll
-  for (int t = 0; t < 4; t++)  // v's 16 columns as B operand
+  for (int cb = 0; cb < NB; cb++) {
 #pragma unroll
-    for (int r = 0; r < 4; r++) {
-      const int i = 16 * t + 4 * r + g;
-      vb[t][r] = i < n ? io.v[i * io.v_ts + (int64_t)h * VD + c0 + i16] : 0.0f;
-    }
-  load_state(S, nkt, l.st, s);
+    for (int t = 0; t < 4; t++)  // v's 16 columns as B operand
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const int i = 16 * t + 4 * r + g;
+        vb[cb][t][r] = i < n ? io.v[i * io.v_ts + (int64_t)h * VD + c0 + VT * cb + i16] : 0.0f;
+      }
+    load_state(S + VT * cb, nkt, s[cb]);
+  }
+  stage_state(l.st, s[0]);
   prep(io, h, 0, n, kv, &l.k[0][0], &l.q[0][0], &l.lp[0][0], &l.tt[0][0], &l.pt[0][0], l.v,
        [&] {
          each_row([&](int i, int d, int j) {
@@ -547,30 +559,44 @@ __global__ __launch_bounds__(CT, 1) void chunk_one(lxm_chunk_io io) {
 #pragma unroll
       for (int r = 0; r < 4; r++) l.w[16 * ti + 4 * g + r][pos16(16 * tc + i16)] = a[r];
     }
-  v4f u = {0.0f, 0.0f, 0.0f, 0.0f};
+  v4f u[NB];
+#pragma unroll
+  for (int cb = 0; cb < NB; cb++) u[cb] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
   for (int t = 0; t < 4; t++) {
-    v4f b;
+    v4f b[NB];
 #pragma unroll
     for (int r = 0; r < 4; r++) {
       const int i = 16 * t + 4 * r + g;
-      b[r] = vb[t][r] * l.v.beta[i];
+#pragma unroll
+      for (int cb = 0; cb < NB; cb++) b[cb][r] = vb[cb][t][r] * l.v.beta[i];
       f[t][r] = l.v.f[i];
     }
     if (t <= w) {
-      u = mfma4(ld_a(&l.tt[0][0], row, 16 * t), b, u);
-      settle(u);
+      const v4f a = ld_a(&l.tt[0][0], row, 16 * t);
+#pragma unroll
+      for (int cb = 0; cb < NB; cb++) {
+        u[cb] = mfma4(a, b[cb], u[cb]);
+        settle(u[cb]);
+      }
     }
   }
   lds_barrier();  // (kb is read: the keys in its place, behind the step's barrier)
   each_row([&](int i, int d, int j) { st4(&l.kb[i][d], kv[j]); });
   const float eg = l.v.eg[row];
-  const v4f o = chunk_step(
-      l.st, &l.kb[0][0], nkt, [&](int t) { return ld4(&l.w[row][16 * t + 4 * g]); },
-      [&](int t) { return ld4(&l.q[row][16 * t + 4 * g]) * eg; }, u, f, l.v.el[0],
-      [&](int t) { return ld_a(&l.a2[0][0], row, 16 * t); }, s, [] {});
-  store_o(io, h, c0, 0, n, o);
-  store_state(S, nkt, s);
+#pragma unroll
+  for (int cb = 0; cb < NB; cb++) {
+    if (cb > 0) {  // (the block before has read its state before its step's barrier, v_new by this one)
+      stage_state(l.st, s[cb]);
+      lds_barrier();
+    }
+    const v4f o = chunk_step(
+        l.st, &l.kb[0][0], nkt, [&](int t) { return ld4(&l.w[row][16 * t + 4 * g]); },
+        [&](int t) { return ld4(&l.q[row][16 * t + 4 * g]) * eg; }, u[cb], f, l.v.el[0],
+        [&](int t) { return ld_a(&l.a2[0][0], row, 16 * t); }, s[cb], [] {});
+    store_o(io, h, c0 + VT * cb, 0, n, o);
+    store_state(S + VT * cb, nkt, s[cb]);
+  }
 }
 
 // q, k, v and S are read four floats at a time: their pointers 16-byte aligned, and the strides
@@ -581,17 +607,26 @@ static bool io_ok(const lxm_chunk_io* io) {
          io->rfull >= io->rl && al16(io->q) && al16(io->k) && al16(io->v) && al16(io->S) &&
          io->qk_ts % 4 == 0 && io->qk_hs % 4 == 0 && io->v_ts % 4 == 0;
 }
-static int cols_grid(int n_slots) { return (n_slots + 7) / 8 * 8 * (VD / VT); }
+static int cols_grid(int n_slots, int nb) { return (n_slots + 7) / 8 * 8 * (VD / (VT * nb)); }
+
+template <int NB>
+static int launch_one(const lxm_chunk_io* io, hipStream_t st) {
+  const int lds = (int)sizeof(OneLds);
+  const hipError_t e = hipFuncSetAttribute((const void*)chunk_one<NB>,
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  if (e != hipSuccess) return (int)e;
+  hipLaunchKernelGGL(chunk_one<NB>, dim3(cols_grid(io->n_slots, NB)), dim3(CT), lds, st, *io);
+  return (int)hipGetLastError();
+}
 
 extern "C" int lxm_gdn_chunk(const lxm_chunk_io* io, void* stream) {
   if (!io_ok(io) || io->n < 1 || io->n > C) return (int)hipErrorInvalidValue;
-  const int lds = (int)sizeof(OneLds);
-  const hipError_t e = hipFuncSetAttribute((const void*)chunk_one,
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-  if (e != hipSuccess) return (int)e;
-  hipLaunchKernelGGL(chunk_one, dim3(cols_grid(io->n_slots)), dim3(CT), lds, (hipStream_t)stream,
-                     *io);
-  return (int)hipGetLastError();
+  // OneLds fills a CU, so a workgroup past the 256th waits for a whole one's time: up to 32 heads 16
+  // columns a workgroup (64 positions of 32 heads 25.1 us), from there on 32, half as many workgroups,
+  // each a step longer (34 heads 29.3 us, 47.2 in 16 columns; 64 heads 29.6 and 48.2; 128 heads 57.1
+  // and 94.4)
+  const bool wide = io->n_slots > 256 / (VD / VT);
+  return wide ? launch_one<2>(io, (hipStream_t)stream) : launch_one<1>(io, (hipStream_t)stream);
 }
 
 extern "C" int lxm_gdn_chunks(const lxm_chunk_io* io, int T, void* ws, int64_t ws_bytes,
@@ -610,7 +645,7 @@ extern "C" int lxm_gdn_chunks(const lxm_chunk_io* io, int T, void* ws, int64_t w
     const int m = nch - c < grp ? nch - c : (int)grp;
     hipLaunchKernelGGL(chunk_prep, dim3(io->n_slots, m), dim3(CT), lds, (hipStream_t)stream, *io, T, c,
                        static_cast<float*>(ws));
-    hipLaunchKernelGGL(chunk_run, dim3(cols_grid(io->n_slots)), dim3(CT), 0, (hipStream_t)stream,
+    hipLaunchKernelGGL(chunk_run, dim3(cols_grid(io->n_slots, 1)), dim3(CT), 0, (hipStream_t)stream,
                        *io, T, c, m, static_cast<const float*>(ws));
   }
   return (int)hipGetLastError();

@@ -121,3 +121,42 @@ def test_chunks_equal_single_chunks(cuda, T, nk, R, kl, groups):
     assert torch.equal(torch.cat(parts), o) and torch.equal(S1, S2)
     assert lib.lxm_gdn_chunks(ctypes.byref(io), T, ctypes.c_void_p(ws.data_ptr()),
                               chunk.CHUNK_WS * nv - 1, None) != 0  # (a workspace too small)
+
+
+@pytest.mark.parametrize("T,nk,R,kl", [(64, 33, 1, 128), (1, 20, 2, 128), (61, 32, 2, 112), (17, 13, 5, 16)])
+def test_chunk_many_heads_equal_few(cuda, T, nk, R, kl):
+    """One chunk of more than 32 value heads (32 state columns a workgroup) leaves the bits of calls of
+    one key head each (16 columns): whole and ragged chunks, head counts off the XCDs' 8."""
+    print(f"[gpu-test] chunk heads T={T} nk={nk} R={R} kl={kl}", flush=True)
+    q, k, v, g, beta, S = (torch.from_numpy(a).to(cuda) for a in _inputs(T, nk, R, 5))
+    q[..., kl:] = 0
+    k[..., kl:] = 0
+    S[:, kl:] = 0
+    S1 = S.clone()
+    o = gated_delta_chunked(q, k, v, g, beta, S1, kl=kl)
+    for h in range(nk):
+        hv = slice(h * R, h * R + R)
+        S2 = S[hv].clone()
+        o2 = gated_delta_chunked(*(t[:, h:h + 1].contiguous() for t in (q, k)),
+                                 *(t[:, hv].contiguous() for t in (v, g, beta)), S2, kl=kl)
+        assert torch.equal(o[:, hv], o2) and torch.equal(S1[hv], S2), h
+
+
+def test_chunk_time_past_one_workgroup_a_cu(cuda):
+    """64 heads' chunk takes no second round of workgroups (32 heads' 16-column ones are one a CU already):
+    1.2 times 32 heads' time, where two rounds are 1.9 times."""
+    us = {}
+    for nk in (16, 32):
+        args = [torch.from_numpy(a).to(cuda) for a in _inputs(64, nk, 2, 3)]
+        best = []
+        for _ in range(20):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            for _ in range(50):
+                gated_delta_chunked(*args)
+            b.record()
+            torch.cuda.synchronize()
+            best.append(a.elapsed_time(b) * 20)
+        us[nk] = min(best)
+    print(f"[gpu-test] chunk of 32 heads {us[16]:.1f} us, of 64 {us[32]:.1f}", flush=True)
+    assert us[32] < 1.5 * us[16], us
