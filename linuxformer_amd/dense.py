@@ -119,7 +119,7 @@ class DenseDecode:
         self.forced = torch.zeros(max_steps, dtype=torch.int32, device=dev)
         self.max_steps = max_steps
         self.graph = None
-        self._pb, self._pb_nt = None, 0
+        self._pb, self._pb_t, self._pb_nt = None, None, 0
 
     def _params(self, n_forced: int, prof: int = 0):
         sp, d = self.spec, self.dims
@@ -148,7 +148,7 @@ class DenseDecode:
             sizes = dict(h=H, xn=H, P=self.nproj, qk=nk * 2 * 256, v=nvr, g=nk * rl * 2,
                          live=nk * 2, o=nvr, ys=nvr, act=I, gl=nk * rl)
             bf = ("xn", "ys", "act")  # (the row kernels' inputs, bf16)
-            self._pb = None  # (the smaller set is given back first)
+            self._pb, self._pb_t, self._pb_nt = None, None, 0  # (the smaller set is freed first)
             self._pb_t = {k: torch.empty(nt * n, device=self.dev,
                                          dtype=torch.bfloat16 if k in bf else torch.float32)
                           for k, n in sizes.items()}

@@ -417,6 +417,45 @@ def test_dense_head_columns_decode_to_the_model(native_lib):
     assert pl0.n_hd == 0 and pl0.summary()["head_dense_cols"] == 0
 
 
+def test_prompt_buffers_grow_without_the_smaller_set(monkeypatch):
+    """A longer prompt's buffers are allocated after the shorter one's are freed (never both at once),
+    a shorter one's calls keep what is there, and a failed allocation leaves none."""
+    import weakref
+
+    import torch
+
+    from linuxformer_amd import dense
+
+    dd = object.__new__(dense.DenseDecode)
+    dd.spec, dd.dev, dd.nproj = synth.config4_small(), "cpu", 3 * 64
+    dd._pb, dd._pb_nt = None, 0
+    refs, live = [], []
+    real = torch.empty
+
+    def empty(*a, **k):
+        live.append(sum(r() is not None for r in refs))
+        return real(*a, **k)
+
+    monkeypatch.setattr(dense.torch, "empty", empty)
+    assert dd._pbuf(3)[1] == 64
+    refs = [weakref.ref(t) for t in dd._pb_t.values()]
+    assert dd._pbuf(64)[1] == 64 and all(r() is not None for r in refs)
+    live.clear()
+    assert dd._pbuf(65)[1] == 128
+    assert live and max(live) == 0
+
+    def full(*a, **k):
+        raise MemoryError
+
+    refs = [weakref.ref(t) for t in dd._pb_t.values()]
+    monkeypatch.setattr(dense.torch, "empty", full)
+    with pytest.raises(MemoryError):
+        dd._pbuf(129)
+    assert not any(r() is not None for r in refs)
+    monkeypatch.setattr(dense.torch, "empty", real)
+    assert dd._pbuf(10)[1] == 64 and dd._pb.h == dd._pb_t["h"].data_ptr()
+
+
 def test_merged_layout_packs_the_chip_rows(native_lib):
     """The chip inside a larger vocabulary (lx/lx/linux.py:108-109's rows = slice(offset,
     offset + VOCAB), Mega's offset): the packed tables equal the chip-only model's, through the
