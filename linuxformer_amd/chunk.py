@@ -22,8 +22,8 @@ WS_MAX = 160 << 20     # a call's workspace at most (68 chunks of 32 heads; more
 def workspace(n_slots: int, T: int, device) -> torch.Tensor:
     """The workspace of a T-position call (lxm_gdn_chunks): every chunk's, or what WS_MAX holds."""
     nch = (T + CHUNK - 1) // CHUNK
-    return torch.empty(n_slots * CHUNK_WS * max(1, min(nch, WS_MAX // (n_slots * CHUNK_WS))),
-                       dtype=torch.uint8, device=device)
+    per = n_slots * CHUNK_WS
+    return torch.empty(per * max(1, min(nch, WS_MAX // max(1, per))), dtype=torch.uint8, device=device)
 
 
 class ChunkIO(ctypes.Structure):

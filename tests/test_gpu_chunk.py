@@ -123,6 +123,13 @@ def test_chunks_equal_single_chunks(cuda, T, nk, R, kl, groups):
                               chunk.CHUNK_WS * nv - 1, None) != 0  # (a workspace too small)
 
 
+@pytest.mark.parametrize("T", [10, 65])
+def test_chunk_refuses_no_heads(cuda, T):
+    z = [torch.zeros(T, *n, device=cuda) for n in ((2, 256), (2, 256), (0, 128), (0,), (0,))]
+    with pytest.raises(RuntimeError, match="hipError"):
+        gated_delta_chunked(*z, torch.zeros(0, 256, 128, device=cuda))
+
+
 @pytest.mark.parametrize("T,nk,R,kl", [(64, 33, 1, 128), (1, 20, 2, 128), (61, 32, 2, 112), (17, 13, 5, 16)])
 def test_chunk_many_heads_equal_few(cuda, T, nk, R, kl):
     """One chunk of more than 32 value heads (32 state columns a workgroup) leaves the bits of calls of

@@ -417,6 +417,16 @@ def test_dense_head_columns_decode_to_the_model(native_lib):
     assert pl0.n_hd == 0 and pl0.summary()["head_dense_cols"] == 0
 
 
+@pytest.mark.parametrize("n_slots,T,chunks", [(0, 65, 0), (0, 1, 0), (1, 64, 1), (32, 65, 2),
+                                              (32, 64 * 69, 68), (3000, 640, 1)])
+def test_chunk_workspace_sizes(n_slots, T, chunks):
+    """Every chunk's workspace, what WS_MAX holds of them, one chunk's at least; none for no heads
+    (the library then refuses the call)."""
+    from linuxformer_amd import chunk
+
+    assert chunk.workspace(n_slots, T, "cpu").numel() == n_slots * chunk.CHUNK_WS * chunks
+
+
 def test_prompt_buffers_grow_without_the_smaller_set(monkeypatch):
     """A longer prompt's buffers are allocated after the shorter one's are freed (never both at once),
     a shorter one's calls keep what is there, and a failed allocation leaves none."""
