@@ -1802,7 +1802,7 @@ __device__ __forceinline__ float conv_b(uint64_t win, const uint16_t* taps, cons
 // query times 1/16, and whether any element is nonzero), the key head's value channels, and its
 // value heads' beta and exp(g), as the step's delta-rule kernel forms them
 __global__ __launch_bounds__(KD) void pb_prep(PbGdn a) {
-  __shared__ float qd[KD], kd[KD];
+  __shared__ float qd[KD], kd[KD], ev[32];
   const int b = blockIdx.x, kh = blockIdx.y, t = tid(), lane = t & 63, wv = t >> 6;
   const int nk = a.nk, kl = a.kl, rl = a.rl, nq = nk * kl, nvr = nk * rl * VD;
   float q = 0.0f, k = 0.0f;
@@ -1828,7 +1828,7 @@ __global__ __launch_bounds__(KD) void pb_prep(PbGdn a) {
     float* g = a.g + ((int64_t)b * nk * rl + vslot) * 2;
     g[0] = bf16r(sigmoid(bb));
     const float gg = (-cr_exp(a.A_log[vh])) * softplus(aa + a.dt_bias[vh]);
-    g[1] = cr_exp(gg);
+    g[1] = ev[t] = cr_exp(gg);
     if (a.gl) a.gl[(int64_t)b * nk * rl + vslot] = gg;
   }
   lds_barrier();
@@ -1857,6 +1857,15 @@ __global__ __launch_bounds__(KD) void pb_prep(PbGdn a) {
     const bool all = __ballot(zero) == 0ull;
     if (lane == 0)
       a.live[((int64_t)b * nk + kh) * 2 + wv] = !any ? 0.0f : all ? 2.0f : 1.0f;
+    // A decay or a key's norm that is not a number reaches the state's zero rows too (0 x NaN in the
+    // step): those pb_gdn<8> leaves alone become NaN here, once any token has one.
+    if (wv && !a.gl && kl <= 128) {
+      for (int r = 0; r < rl; r++) {
+        if (ev[r] == ev[r] && inv == inv) continue;
+        float* S = a.rec + ((size_t)(kh * a.R + r) * KD + 128) * VD;
+        for (int i = lane; i < (KD - 128) * VD; i += 64) S[i] = __builtin_nanf("");
+      }
+    }
   }
 }
 // x summed over the NB lanes of a column in lane order, on every one of them: lane b adds its left
@@ -1885,7 +1894,7 @@ __device__ __forceinline__ float col_spread(float a) {
 // The delta rule over the batch's tokens in order: a one-wave workgroup holds 64 / NB columns of one
 // live value head's state, lane c NB + b rows 16 b .. 16 b + 15 of column c (one of ATen's
 // 16-row cascade blocks), NB = 8 blocks where the live key dims end at 128 (the rows past them are
-// zero and stay so), else 16. A token is a serial chain of ~140 vector ops: the block's dot with k, the
+// zero and stay so, or become NaN in pb_prep), else 16. A token is a serial chain of ~140 vector ops: the block's dot with k, the
 // blocks in order across the column's lanes, the update, the dot with q. No barrier and no
 // LDS: a lane's 16 key and query values come from memory (L2) three tokens ahead, in four fixed
 // buffers. A head's waves go to one XCD, which then holds its queries and keys in its L2. Bound by the

@@ -179,6 +179,52 @@ def test_dense_prefill_key_dims(cuda, kl, zeros):
     assert (bits(cache.rec_numpy()) == bits(r)).all()
 
 
+@pytest.mark.parametrize("kl", [64, 128, 160])
+@pytest.mark.parametrize("kind", ["key", "decay", "value", "large"])
+def test_dense_prefill_not_finite(cuda, kl, kind):
+    """Weights that make a key, a decay or a value NaN or infinite, and products that overflow: the live
+    heads' states and windows are NaN where the oracle's are (a NaN key or decay reaches the zero rows
+    past the live key dims, a value only its column) and its bits elsewhere."""
+    from dataclasses import replace
+
+    from oracle import oracle as ox
+
+    spec = replace(synth.config4_small(), kd_live=kl)
+    dm = synth.build_dense(spec, "cpu")
+    conv0, rec0 = synth.dense_state(dm, 3)
+    ly = dm.layers[0]
+    if kind == "key":
+        ly["qk"][1, 1, 3, 5] = float("nan")
+    elif kind == "decay":
+        ly["a"][0, 1, 7] = float("nan")
+    elif kind == "value":
+        ly["v"][0, 0, 3, 5] = float("inf")
+    else:
+        for ly in dm.layers:
+            for n in ("qk", "v", "z", "b", "a", "out", "gate", "up", "down"):
+                ly[n] = (ly[n].float() * 1e30).bfloat16()
+    toks = [int(x) for x in np.random.default_rng(29).integers(0, spec.vocab, 21)]
+    print(f"[gpu-test] dense prefill not finite: kl={kl} {kind}", flush=True)
+    cache = fast.StateCache(conv0, rec0, "bf16", "cuda")
+    dense.DenseDecode(synth.dense_to(dm, "cuda"), cache).prefill(toks)
+    c, r = conv0.copy(), rec0.copy()
+    ox.OracleModel(synth.to_sparse(dm)).decode(c, r, toks, len(toks))
+    # (the dead heads and channels: the kernels leave them alone, the oracle's 0 x NaN does not)
+    R = spec.nv // spec.nk
+
+    def live(conv, rec):
+        rec = rec.reshape(-1, spec.nk, R, 256, 128)[:, :, :spec.r_live]
+        nq = 2 * spec.nk * 256
+        qk = conv[:, :nq].reshape(-1, 2 * spec.nk, 256, 4)[:, :, :kl]
+        return rec, qk, conv[:, nq:].reshape(-1, spec.nk, R, 128, 4)[:, :, :spec.r_live]
+
+    got, want = live(cache.conv_numpy(), cache.rec_numpy()), live(c, r)
+    assert any(np.isnan(w).any() for w in want)
+    for x, y in zip(got, want):
+        assert (np.isnan(x) == np.isnan(y)).all()
+        assert (bits(x)[~np.isnan(y)] == bits(y)[~np.isnan(y)]).all()
+
+
 @pytest.mark.parametrize("n", [5, 40])
 def test_dense_prefill_repeats(cuda, n):
     """The same prompt twice leaves the same bits at the full row lengths (a short prompt's kernels
