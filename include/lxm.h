@@ -188,6 +188,10 @@ int lxm_t_elem(int fn, const float* x, float* y, long n, void* stream);
 /* kind 0: the 512-lane hidden sum, kind 1: the 64-lane head sum, of each of rows rows of n
    values (x row-major); out (rows). */
 int lxm_t_sum(int kind, const float* x, int n, int rows, float* out, void* stream);
+/* The fp32 matrix instructions' sums: out (rows x rows) = the chains over k = 0 .. K - 1 from +0 of
+   a[i][k] b[j][k] (a, b: rows x K), rows 32 (v_mfma_f32_32x32x2_f32) or 16 (v_mfma_f32_16x16x4_f32);
+   K a multiple of 4, at most 4096. */
+int lxm_t_mfma(int rows, const float* a, const float* b, int K, float* out, void* stream);
 
 /* No counterpart in the reference: lxm_run for callers that cannot allocate device memory (tight
    serving loops, harnesses that forbid hipMalloc). It is a cooperative launch, which is not

@@ -1366,9 +1366,9 @@ __device__ __forceinline__ uint16_t bf16_bits(float v) { return (uint16_t)(fbits
 // Rows for a batch of n tokens on the fp32 matrix cores, in the step's order. The order of a dense
 // row is 64 groups of G entries, each summed in order from +0, then the pairwise tree over the
 // groups. v_mfma_f32_32x32x2_f32 accumulates its two k in order, each step one fused
-// multiply-add rounded to nearest even with denormals kept (checked against a host fmaf chain in
-// seven regimes of magnitude), and bf16 x bf16 products are exact in fp32: a group's chain of MFMAs
-// from zero is its sum, bit for bit, for 32 rows x 32 tokens at once.
+// multiply-add rounded to nearest even with denormals kept (lxm_t_mfma; the tests hold it to host chains
+// of fused multiply-adds in eight regimes of magnitude), and bf16 x bf16 products are exact in fp32: a
+// group's chain of MFMAs from zero is its sum, bit for bit, for 32 rows x 32 tokens at once.
 //
 // A workgroup (4 waves) takes 32 rows x 64 tokens. Its waves split the groups, not the tile: wave
 // w takes the groups congruent to w mod 4, so one step stages 4 consecutive groups' chunk q (64

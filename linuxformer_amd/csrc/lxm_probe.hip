@@ -1,3 +1,6 @@
+// What the other kernels rest on, by itself: cross-workgroup synchronisation costs (lxm_t_sync), and the
+// sums of the fp32 matrix instructions (lxm_t_mfma).
+//
 // Cross-workgroup synchronisation costs on MI355X, measured with the primitives the decode and
 // dense kernels use (lxm_sync.h): agent-scope relaxed words polled by one thread per workgroup
 // with the same bounded spin (s_sleep between polls, a 3 s wall-clock limit that sets the error
@@ -64,7 +67,38 @@ __global__ void __launch_bounds__(64) k_sync(int kind, int n_iter, int far, uint
   if (b == 0) out[0] = ok ? (float)(wall() - t0) * 0.01f / (float)n_iter : -1.0f;
 }
 
+// One wave: out[i][j] = the chain over k from +0 of a[i][k] b[j][k], R rows of each, as the dense prompt's
+// row kernels issue it (R = 32: two k an instruction, 16: four)
+typedef float v16f __attribute__((ext_vector_type(16)));
+template <int R>
+__global__ void __launch_bounds__(64) k_mfma(const float* a, const float* b, int K, float* out) {
+  constexpr int KI = 64 / R;  // k per instruction
+  const int lane = threadIdx.x, i = lane % R, k0 = lane / R;
+  if constexpr (R == 32) {
+    v16f c = {0};
+    for (int k = 0; k < K; k += KI)
+      c = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i * K + k + k0], b[i * K + k + k0], c, 0, 0, 0);
+#pragma unroll
+    for (int r = 0; r < 16; r++) out[(8 * (r / 4) + 4 * k0 + r % 4) * R + i] = c[r];
+  } else {
+    v4f c = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int k = 0; k < K; k += KI)
+      c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i * K + k + k0], b[i * K + k + k0], c, 0, 0, 0);
+#pragma unroll
+    for (int r = 0; r < 4; r++) out[(4 * k0 + r) * R + i] = c[r];
+  }
+}
+
 }  // namespace
+
+extern "C" int lxm_t_mfma(int rows, const float* a, const float* b, int K, float* out, void* stream) {
+  if ((rows != 32 && rows != 16) || K < 4 || K % 4 || K > 4096 || !a || !b || !out)
+    return (int)hipErrorInvalidValue;
+  const hipStream_t st = (hipStream_t)stream;
+  if (rows == 32) hipLaunchKernelGGL(k_mfma<32>, dim3(1), dim3(64), 0, st, a, b, K, out);
+  else hipLaunchKernelGGL(k_mfma<16>, dim3(1), dim3(64), 0, st, a, b, K, out);
+  return (int)hipGetLastError();
+}
 
 extern "C" int lxm_t_sync(int kind, int n_iter, int n_blocks, int far, uint32_t* words,
                           int32_t* err, float* out_us, void* stream) {

@@ -97,6 +97,8 @@ def load(subprof: bool = False) -> ctypes.CDLL:
         lib.lxm_t_elem.restype = I
         lib.lxm_t_sum.argtypes = [I, P, I, I, P, P]
         lib.lxm_t_sum.restype = I
+        lib.lxm_t_mfma.argtypes = [I, P, P, I, P, P]
+        lib.lxm_t_mfma.restype = I
         lib.lxm_helper_lds.argtypes = [I]
         lib.lxm_helper_lds.restype = I
         for n in ("lxm_pf_head", "lxm_pf_embed"):
@@ -129,7 +131,7 @@ def load(subprof: bool = False) -> ctypes.CDLL:
 
 
 EXPORTS = ("lxm_run", "lxm_lds_base", "lxm_helper_lds", "lxm_max_blocks", "lxm_max_lds",
-           "lxm_last_error", "lxm_device_cus", "lxm_t_elem", "lxm_t_sum", "lxm_pf_layers",
+           "lxm_last_error", "lxm_device_cus", "lxm_t_elem", "lxm_t_sum", "lxm_t_mfma", "lxm_pf_layers",
            "lxm_pf_head", "lxm_pf_embed", "lxm_pf_tiles", "lxm_pf_lds", "lxm_dn_step", "lxm_dn_run",
            "lxm_dn_prefill", "lxm_t_sync", "lxm_run_noalloc", "lxm_gdn_chunk",
            "lxm_dn_prefill_chunked", "lxm_dn_prefill_n", "lxm_gdn_chunks")

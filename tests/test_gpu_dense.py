@@ -283,8 +283,135 @@ def test_dense_prefill_batches(cuda, chunked, nt):
         assert (bits(a) == bits(b)).all()
 
 
+def fma_chain(a, b):
+    """sum_k a[:, k] b[:, k]' from +0 in k order, each step one fused multiply-add rounded to the nearest
+    even float32, denormals kept: products of float32 are exact in float64; the sum is rounded to odd
+    there (53 bits), so the rounding to 24 is the only one."""
+    acc = np.zeros((a.shape[0], b.shape[0]), np.float32)
+    for k in range(a.shape[1]):
+        p = a[:, k].astype(np.float64)[:, None] * b[:, k].astype(np.float64)[None]
+        c = acc.astype(np.float64)
+        s = c + p
+        t = s - c
+        e = (c - (s - t)) + (p - t)
+        odd = np.isfinite(s) & np.isfinite(e) & (e != 0) & (s.view(np.uint64) & 1 == 0)
+        s = np.where(odd, np.nextafter(s, np.where(e > 0, np.inf, -np.inf)), s)
+        acc = s.astype(np.float32)
+    return acc
+
+
+REGIMES = ["normal", "wide", "cancel", "denormal_in", "denormal_out", "overflow", "not_finite",
+           "float32"]
+
+
+@pytest.mark.parametrize("rows", [32, 16])
+@pytest.mark.parametrize("regime", REGIMES)
+@np.errstate(all="ignore")
+def test_mfma_sums_are_fma_chains(cuda, rows, regime):
+    """What the prompt's row kernels rest on: the fp32 matrix instructions add their k in order, each step
+    one fused multiply-add, denormals kept, from +0: bit for bit at the kernels' chain lengths (one group's
+    4 to 144 entries), in regimes of magnitude."""
+    import ctypes
+
+    libm = ctypes.CDLL("libm.so.6")
+    libm.fmaf.argtypes, libm.fmaf.restype = [ctypes.c_float] * 3, ctypes.c_float
+    rng = np.random.default_rng(rows * 10 + REGIMES.index(regime))
+    print(f"[gpu-test] mfma chains rows={rows} {regime}", flush=True)
+    seen = np.zeros(0, np.float32)
+    for K in (4, 8, 40, 64, 144):
+        for _ in range(6):
+            a, b = (rng.standard_normal((rows, K)) for _ in range(2))
+            if regime == "wide":
+                a, b = (x * 2.0 ** rng.integers(-45, 46, x.shape) for x in (a, b))
+            elif regime == "cancel":  # (each pair of terms nearly cancels)
+                a[:, 1::2] = -a[:, ::2]
+                b[:, 1::2] = b[:, ::2] * (1 + 2.0 ** -7 * rng.integers(-1, 2, b[:, ::2].shape))
+            elif regime == "denormal_in":
+                a, b = a * 2.0 ** -128, b * 2.0 ** rng.integers(-2, 100, b.shape)
+            elif regime == "denormal_out":
+                a, b = (x * 2.0 ** rng.integers(-75, -63, x.shape) for x in (a, b))
+            elif regime == "overflow":
+                a, b = (x * 2.0 ** rng.integers(58, 65, x.shape) for x in (a, b))
+            elif regime == "not_finite":
+                a[0, 1], b[1, 2], a[2, 3], b[2, 3] = np.inf, -np.inf, np.nan, 0.0
+            a, b = a.astype(np.float32), b.astype(np.float32)
+            if regime != "float32":
+                a, b = (torch.from_numpy(x).bfloat16().float().numpy() for x in (a, b))
+            want = fma_chain(a, b)
+            x = np.float32(0)
+            for k in range(K):
+                x = libm.fmaf(float(a[3, k]), float(b[2, k]), float(x))
+            assert bits(np.float32(x)) == bits(want[3, 2]) or np.isnan(x)
+            ad, bd = torch.from_numpy(a).to(cuda), torch.from_numpy(b).to(cuda)
+            out = torch.zeros(rows, rows, device=cuda)
+            assert mk_build.load().lxm_t_mfma(rows, ctypes.c_void_p(ad.data_ptr()),
+                                              ctypes.c_void_p(bd.data_ptr()), K,
+                                              ctypes.c_void_p(out.data_ptr()), None) == 0
+            got = out.cpu().numpy()
+            assert ((bits(got) == bits(want)) | (np.isnan(got) & np.isnan(want))).all(), K
+            seen = np.concatenate([seen, (a if regime == "denormal_in" else want).reshape(-1)])
+    mag = np.abs(seen)
+    if regime.startswith("denormal"):  # (the regime is what it says)
+        assert ((mag > 0) & (mag < 2.0 ** -126)).mean() > 0.01
+    if regime == "overflow":
+        assert 0.01 < np.isinf(seen).mean() < 0.99
+    if regime == "not_finite":
+        assert np.isnan(seen).any() and np.isinf(seen).any()
+
+
 def test_dense_prefill_full_widths(cuda):
     check_prefill(21, 3, seed=5, name="mid")
+
+
+TWO_LAYERS = [9, 25, 40, 70]  # prompt lengths
+
+
+@pytest.fixture(scope="module")
+def wide():
+    """Two layers at config 4's full widths (layer 1's states see layer 0's out_proj, SwiGLU and
+    down_proj), and the oracle's states after each of the prompts below."""
+    from dataclasses import replace
+
+    from oracle import oracle as ox
+
+    spec = replace(synth.config4_mid(), n_layers=2, vocab=256)
+    dm = synth.build_dense(spec, "cpu")
+    conv0, rec0 = synth.dense_state(dm, 5)
+    toks = [int(x) for x in np.random.default_rng(41).integers(0, spec.vocab, 200)]
+    om = ox.OracleModel(synth.to_sparse(dm))
+    c, r, at, done = conv0.copy(), rec0.copy(), {}, 0
+    for n in TWO_LAYERS:
+        print(f"[gpu-test] the oracle's tokens {done} .. {n - 1}", flush=True)
+        om.decode(c, r, toks[done:n], n - done)
+        at[n], done = (c.copy(), r.copy()), n
+    return synth.dense_to(dm, "cuda"), conv0, rec0, toks, at
+
+
+@pytest.mark.parametrize("n", TWO_LAYERS)
+def test_dense_prefill_full_widths_two_layers(cuda, wide, n):
+    """Every row kernel at its real row lengths against the oracle, seen through layer 1: 16-row tiles of 16,
+    32 and (hidden rows) 64 tokens, 32-row tiles with a whole and a partial token tile."""
+    dm, conv0, rec0, toks, at = wide
+    print(f"[gpu-test] dense prefill two full-width layers: n={n}", flush=True)
+    cache = fast.StateCache(conv0, rec0, "bf16", "cuda")
+    dense.DenseDecode(dm, cache).prefill(toks[:n])
+    assert (bits(cache.conv_numpy()) == bits(at[n][0])).all()
+    assert (bits(cache.rec_numpy()) == bits(at[n][1])).all()
+
+
+@pytest.mark.parametrize("n", [64, 65, 130, 200])
+def test_dense_prefill_full_widths_equals_steps(cuda, wide, n):
+    """More token tiles: the states of as many forced steps."""
+    dm, conv0, rec0, toks, _ = wide
+    print(f"[gpu-test] dense prefill two full-width layers against steps: n={n}", flush=True)
+    out = []
+    for batched in (False, True):
+        cache = fast.StateCache(conv0, rec0, "bf16", "cuda")
+        dd = dense.DenseDecode(dm, cache, max_steps=256)
+        dd.prefill(toks[:n]) if batched else dd.run(toks[:n], n)
+        out.append((cache.conv_numpy(), cache.rec_numpy()))
+    for a, b in zip(*out):
+        assert (bits(a) == bits(b)).all()
 
 
 def test_dense_prefill_equals_steps_config4(cuda):
