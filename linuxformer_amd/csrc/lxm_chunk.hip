@@ -21,7 +21,8 @@
 // A chunk's chain is bound by its latency: a wave's two products of 32 MFMAs, a barrier, a triangular one
 // and one of 32, a barrier, where one workgroup per (head, chunk, 32 columns)
 // and a launch a chunk took 31 us, each column block repeating the inverse. 2,048 positions of 32 heads:
-// 1,020 -> 234 us (chunk_prep 68, chunk_run 179: 5.6 a chunk); 100 positions of 4 heads 62.3 -> 34.4.
+// 1,020 -> 234 us (under a kernel trace, which adds to both, chunk_prep 67 and chunk_run 179: 5.6 a
+// chunk); 100 positions of 4 heads 62.3 -> 34.4.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -355,7 +356,9 @@ __device__ __forceinline__ v4f chunk_step(StepLds& st, const float* k, int nkt, 
 __device__ __forceinline__ float* state_of(const lxm_chunk_io& io, int h, int c0) {
   return io.S + ((size_t)(h / io.rl) * io.rfull + h % io.rl) * 256 * VD + c0;
 }
-__device__ __forceinline__ void load_state(const float* S, int nkt, v4f (&s)[2]) {
+// (STAGE: each tile into st.s as it comes)
+template <bool STAGE>
+__device__ __forceinline__ void load_state(const float* S, int nkt, StepLds& st, v4f (&s)[2]) {
   const int w = wave(), lane = threadIdx.x & 63, i16 = lane & 15, g = lane >> 4;
 #pragma unroll
   for (int j = 0; j < 2; j++) {
@@ -364,12 +367,8 @@ __device__ __forceinline__ void load_state(const float* S, int nkt, v4f (&s)[2])
 #pragma unroll
       for (int r = 0; r < 4; r++) s[j][r] = S[(size_t)(16 * (2 * w + j) + 4 * g + r) * VD + i16];
     }
+    if constexpr (STAGE) st_b(st.s[2 * w + j], s[j]);
   }
-}
-__device__ __forceinline__ void stage_state(StepLds& st, const v4f (&s)[2]) {
-  const int w = wave();
-#pragma unroll
-  for (int j = 0; j < 2; j++) st_b(st.s[2 * w + j], s[j]);
 }
 __device__ __forceinline__ void store_state(float* S, int nkt, const v4f (&s)[2]) {
   const int w = wave(), lane = threadIdx.x & 63, i16 = lane & 15, g = lane >> 4;
@@ -482,8 +481,7 @@ __global__ __launch_bounds__(CT, 1) void chunk_run(lxm_chunk_io io, int T, int c
     }
     el = x[WS_V + 2 * C];
   };
-  load_state(S, nkt, s);
-  stage_state(l.st, s);
+  load_state<true>(S, nkt, l.st, s);
   get_kq(0);
   get_rest(0);
   lds_barrier();
@@ -541,9 +539,9 @@ __global__ __launch_bounds__(CT, 1) void chunk_one(lxm_chunk_io io) {
         const int i = 16 * t + 4 * r + g;
         vb[cb][t][r] = i < n ? io.v[i * io.v_ts + (int64_t)h * VD + c0 + VT * cb + i16] : 0.0f;
       }
-    load_state(S + VT * cb, nkt, s[cb]);
+    if (cb == 0) load_state<true>(S, nkt, l.st, s[0]);
+    else load_state<false>(S + VT * cb, nkt, l.st, s[cb]);
   }
-  stage_state(l.st, s[0]);
   prep(io, h, 0, n, kv, &l.k[0][0], &l.q[0][0], &l.lp[0][0], &l.tt[0][0], &l.pt[0][0], l.v,
        [&] {
          each_row([&](int i, int d, int j) {
@@ -587,7 +585,8 @@ __global__ __launch_bounds__(CT, 1) void chunk_one(lxm_chunk_io io) {
 #pragma unroll
   for (int cb = 0; cb < NB; cb++) {
     if (cb > 0) {  // (the block before has read its state before its step's barrier, v_new by this one)
-      stage_state(l.st, s[cb]);
+#pragma unroll
+      for (int j = 0; j < 2; j++) st_b(l.st.s[2 * w + j], s[cb][j]);
       lds_barrier();
     }
     const v4f o = chunk_step(

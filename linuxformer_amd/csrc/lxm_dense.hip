@@ -1894,10 +1894,10 @@ __device__ __forceinline__ float col_spread(float a) {
 // The delta rule over the batch's tokens in order: a one-wave workgroup holds 64 / NB columns of one
 // live value head's state, lane c NB + b rows 16 b .. 16 b + 15 of column c (one of ATen's
 // 16-row cascade blocks), NB = 8 blocks where the live key dims end at 128 (the rows past them are
-// zero and stay so, or become NaN in pb_prep), else 16. A token is a serial chain of ~140 vector ops: the block's dot with k, the
-// blocks in order across the column's lanes, the update, the dot with q. No barrier and no
-// LDS: a lane's 16 key and query values come from memory (L2) three tokens ahead, in four fixed
-// buffers. A head's waves go to one XCD, which then holds its queries and keys in its L2. Bound by the
+// zero and stay so, or become NaN in pb_prep), else 16. A token is a serial chain of ~140 vector
+// ops: the block's dot with k, the blocks in order across the column's lanes, the update, the dot
+// with q. No barrier and no LDS: a lane's 16 key and query values come from memory (L2) three tokens
+// ahead, in four fixed buffers. A head's waves go to one XCD, which then holds its queries and keys in its L2. Bound by the
 // chain's issue (148 vector ops a token): 0.49 us a token and layer at 32 live heads of 128 key dims,
 // where 8-wave workgroups of 32 columns, whose sums crossed waves through LDS (three barriers a
 // token), took 1.66. No faster: this token's query dot interleaved with the next one's key dot (0.56),

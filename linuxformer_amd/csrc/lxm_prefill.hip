@@ -866,7 +866,7 @@ __device__ __forceinline__ void tail_chan(const lxm_pf_params& p, const lxm_pf_l
 #define KQ_Q (20 * KD / 16)  // the q half of a wave's k and q staging
 // A candidate's inputs as one lane holds them (loaded three candidates ahead): the header word,
 // the slot's decay factor, its column's v, beta, and an eighth of the slot's k and q (lanes
-// 0-31 k, 32-63 q, 8 values each), which the step stages in the wave's LDS for every lane.
+// 0-31 k, 32-63 q, 8 values each), which the step before stages in the wave's LDS for every lane.
 struct DeltaIn {
   uint32_t live;
   float e, v, beta;
@@ -1045,10 +1045,10 @@ __global__ __launch_bounds__(64) void pf_delta(const lxm_pf_params* __restrict__
 // pairwise tree, one wave per head. Then out_proj and the residual add at the candidate
 // (TF:541-543, :777-779): per residual row the terms over every value dim in ascending order,
 // rounded once (lx/lx/fast.py:349-361), then h = D(h + that). Heads that did not run add nothing
-// (their output is exactly 0 and the oracle skips zero inputs). One workgroup per candidate.
-// parts_of() workgroups share a candidate's residual rows, each forming the norms; a wave's heads come
-// four at a time, their inputs requested together (one workgroup a candidate, a head at a time: 15.2 us
-// a layer at 61 positions, 8.6 now).
+// (their output is exactly 0 and the oracle skips zero inputs). parts_of() workgroups share a
+// candidate's residual rows, each forming the norms; a wave's heads come four at a time, their inputs
+// requested together (one workgroup a candidate, a head at a time: 15.2 us a layer at 61 positions, 8.3
+// now).
 template <bool BF>
 __global__ __launch_bounds__(NT) void pf_out(const lxm_pf_params* __restrict__ pp, int L) {
   extern __shared__ __align__(16) uint8_t sm[];
