@@ -109,10 +109,10 @@ typedef struct lxm_dn_pbuf {
 /* T forced tokens (device int32) through every layer without the head, in batches of LXM_DN_PB:
    the states and windows afterwards are those T calls of lxm_dn_step with these forced tokens
    leave, bit for bit (each weight row is read once per 64 tokens of a batch; every sum keeps the
-   step's order; lxm_dn_prefill_n takes larger batches). The stock generate's prefill role (the prompt before the first prediction, here with
-   the decode's per-token arithmetic); a caller then steps from the next token. A token out of
-   range sets *err = 1 (row 0 is used). Supports (hidden, live value dims, inter) = (2560, 4096,
-   9216) or (256, 512, 512). Returns a hipError_t. */
+   step's order; lxm_dn_prefill_n takes larger batches). The stock generate's prefill role (the
+   prompt before the first prediction, here with the decode's per-token arithmetic); a caller then
+   steps from the next token. A token out of range sets *err = 1 (row 0 is used). Supports (hidden,
+   live value dims, inter) = (2560, 4096, 9216) or (256, 512, 512). Returns a hipError_t. */
 int lxm_dn_prefill(const lxm_dn_params* p_host, const int32_t* tokens, int T,
                    const lxm_dn_pbuf* buf, void* stream);
 
@@ -132,9 +132,9 @@ int lxm_dn_prefill_chunked(const lxm_dn_params* p_host, const int32_t* tokens, i
 /* Both prompts with buffers of nt tokens (buf's arrays hold nt tokens each: the sizes above with
    PB = nt): lxm_dn_prefill's results (chunked 0) or lxm_dn_prefill_chunked's (chunked 1; nt a
    multiple of LXM_CHUNK, buf->gl set, and past one chunk a workspace ws of ws_bytes as
-   lxm_gdn_chunks takes it for nk x rl slots; else ws may be null), in batches of nt tokens. A batch's rows run on the matrix
-   cores at any nt with the same bits; a larger nt reads each weight row fewer times. Returns a
-   hipError_t. */
+   lxm_gdn_chunks takes it for nk x rl slots; else ws may be null), in batches of nt tokens. A
+   batch's rows run on the matrix cores at any nt with the same bits; a larger nt reads each weight
+   row fewer times. Returns a hipError_t. */
 int lxm_dn_prefill_n(const lxm_dn_params* p_host, const int32_t* tokens, int T,
                      const lxm_dn_pbuf* buf, int nt, int chunked, void* ws,
                      int64_t ws_bytes, void* stream);

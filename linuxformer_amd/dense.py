@@ -161,11 +161,11 @@ class DenseDecode:
         then steps from the next token: run([next], n).
 
         mode "batched" (lxm_dn_prefill_n: batches of up to NT_MAX tokens, each layer's products on
-        the matrix cores in the step's order): the cache's states and windows afterwards are those of len(tokens) forced steps
-        of run(), bit for bit. mode "chunked": the stock forward's
-        T > 1 path, the delta rule in chunks of 64 on the matrix cores
-        (torch_chunk_gated_delta_rule); every other sum as in "batched", the delta rule's outputs
-        and states those of the chunked form."""
+        the matrix cores in the step's order): the cache's states and windows afterwards are those
+        of len(tokens) forced steps of run(), bit for bit. mode "chunked": the stock forward's T > 1
+        path, the delta rule in chunks of 64 on the matrix cores (torch_chunk_gated_delta_rule);
+        every other sum as in "batched", the delta rule's outputs and states those of the chunked
+        form. The buffers of the longest prompt so far (up to NT_MAX tokens) are kept."""
         if mode not in ("batched", "chunked"):
             raise ValueError(f"prefill mode {mode!r}: 'batched' or 'chunked'")
         t = torch.as_tensor(tokens, dtype=torch.int64)
