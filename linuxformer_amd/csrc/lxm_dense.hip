@@ -1859,7 +1859,8 @@ __global__ __launch_bounds__(KD) void pb_prep(PbGdn a) {
       a.live[((int64_t)b * nk + kh) * 2 + wv] = !any ? 0.0f : all ? 2.0f : 1.0f;
     // A decay or a key's norm that is not a number reaches the state's zero rows too (0 x NaN in the
     // step): those pb_gdn<8> leaves alone become NaN here, once any token has one.
-    if (wv && !a.gl && kl <= 128) {
+    const float e = ev[lane < rl ? lane : 0];
+    if (wv && !a.gl && kl <= 128 && (__ballot(e != e) != 0ull || inv != inv)) {
       for (int r = 0; r < rl; r++) {
         if (ev[r] == ev[r] && inv == inv) continue;
         float* S = a.rec + ((size_t)(kh * a.R + r) * KD + 128) * VD;
